@@ -221,6 +221,12 @@ __device__ __forceinline__ uint16_t swiglu_out(float up, float gate)
     return f2h(h2f(f2h(up)) * h2f(f2h(silu(gate))));
 }
 
+// the FFN_UP_AND_GATE op's result from the fp32 sums (src/shaders/vkllm_ffn_up_and_gate.comp:133-147)
+__device__ __forceinline__ uint16_t ffn_out(float up, float gate)
+{
+    return f2h(up * gate / (1.0f + expf(-gate)));
+}
+
 // Prompt-step activations of at most 128 rows (tokens) kept in the operand order of v_mfma_f32_32x32x16_f16's B
 // matrix over 32-token blocks, so a wave reads one 16-K step of one token block as 1 KB contiguous: the 16-byte
 // vector holding row t, columns 8 kv .. 8 kv + 7 of an [M <= 128, K] fp16 matrix is vector number

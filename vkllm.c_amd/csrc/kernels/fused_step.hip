@@ -274,6 +274,8 @@ template <int EPI> __device__ __forceinline__ void gemv_rows_of(const GemvArgs &
     {
         if (EPI == EPI_GATEUP)
             rows[k] = k < R / 2 ? (R / 2) * u + k : a.rows / 2 + (R / 2) * u + (k - R / 2);
+        else if (EPI == EPI_FFN) // row k of w, then the same row of w2
+            rows[k] = (R / 2) * u + k % (R / 2);
         else
             rows[k] = R * u + k;
     }
@@ -308,6 +310,13 @@ template <int EPI, int R> __device__ __forceinline__ void gemv_epilogue(const Ge
             const float gate = h2f(f2h(silu(acc[k + R / 2])));
             a.out[(R / 2) * u + k] = f2h(up * gate);
         }
+    }
+    else if (EPI == EPI_FFN)
+    {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k)
+            if (rows[k] < a.rows)
+                a.out[rows[k]] = ffn_out(acc[k], acc[k + R / 2]);
     }
     else // EPI_QKV: rows (r, r + 1), r even, are one RoPE pair of one head
     {
@@ -358,10 +367,10 @@ template <int EPI, int R> __device__ __forceinline__ void gemv_epilogue(const Ge
     }
 }
 
-// the epilogues whose input is the RMSNorm of the residual stream (all but the residual products)
+// the epilogues whose input is the RMSNorm of the residual stream (all but the residual products and the operators)
 constexpr bool gemv_normalises(int epi)
 {
-    return epi != EPI_RESID && epi != EPI_RAW;
+    return epi != EPI_RESID && epi != EPI_RAW && epi != EPI_FFN;
 }
 
 // EPI_QKV_ATTN's tail, all 256 threads of the workgroup: single-token attention of head `head` over kv positions
@@ -583,7 +592,8 @@ template <int EPI, int R, int NV> __global__ __launch_bounds__(256) void gemv_fa
         {
             // rows past the end (or of units past the end) read row 0; their sums are never stored
             const bool ok = unit < units && rows[k] < a.rows;
-            const u32x4 *wr = (const u32x4 *)(a.w + (size_t)(ok ? rows[k] : 0) * a.K);
+            const uint16_t *wb = EPI == EPI_FFN && k >= R / 2 ? a.w2 : a.w;
+            const u32x4 *wr = (const u32x4 *)(wb + (size_t)(ok ? rows[k] : 0) * a.K);
 #pragma unroll
             for (int i = 0; i < NV; ++i)
                 w[k][i] = __builtin_nontemporal_load(wr + min(lane + 64 * i, nvec - 1));
@@ -795,8 +805,10 @@ static uint32_t gemv_units(int epi, const GemvArgs &a, int R)
 {
     if (epi == EPI_GATEUP)
         return (R % 2 == 0 && a.rows % R == 0) ? a.rows / R : 0;
-    if (is_qkv(epi) && R % 2 != 0)
+    if ((is_qkv(epi) || epi == EPI_FFN) && R % 2 != 0)
         return 0;
+    if (epi == EPI_FFN) // R / 2 rows of each of the two matrices
+        return (a.rows + R / 2 - 1) / (R / 2);
     return (a.rows + R - 1) / R;
 }
 
@@ -896,7 +908,7 @@ static hipError_t launch_argmax_epi(hipStream_t st, const GemvArgs &a, int cu_co
 static int gemv_default_r(int epi, uint32_t K)
 {
     (void)K;
-    return epi == EPI_GATEUP || is_qkv(epi) ? 2 : 1;
+    return epi == EPI_GATEUP || epi == EPI_FFN || is_qkv(epi) ? 2 : 1;
 }
 
 hipError_t launch_gemv(hipStream_t st, int epi, const GemvArgs &a, int cu_count)
@@ -905,7 +917,7 @@ hipError_t launch_gemv(hipStream_t st, int epi, const GemvArgs &a, int cu_count)
         return hipErrorInvalidValue;
     const uint32_t nvec = a.K / 8;
     int R = a.rows_per_unit ? (int)a.rows_per_unit : gemv_default_r(epi, a.K);
-    if (R == 1 && (epi == EPI_GATEUP || is_qkv(epi)))
+    if (R == 1 && (epi == EPI_GATEUP || epi == EPI_FFN || is_qkv(epi)))
         R = 2;
     // the attention tail: a head's V row as 4 to 64 16-byte vectors (a lane each)
     if (epi == EPI_QKV_ATTN && (R != 2 || a.H > kAttnTailMaxHeads || a.hd % 8 != 0 || a.hd < 32 ||
@@ -937,6 +949,8 @@ hipError_t launch_gemv(hipStream_t st, int epi, const GemvArgs &a, int cu_count)
             return launch_epi<EPI_RESID>(st, a, cu_count, R, NV);
         case EPI_GATEUP:
             return launch_epi<EPI_GATEUP>(st, a, cu_count, R, NV);
+        case EPI_FFN:
+            return a.w2 ? launch_epi<EPI_FFN>(st, a, cu_count, R, NV) : hipErrorInvalidValue;
         case EPI_QKV:
             return launch_epi<EPI_QKV>(st, a, cu_count, R, NV);
         case EPI_QKV_ATTN:
@@ -947,7 +961,8 @@ hipError_t launch_gemv(hipStream_t st, int epi, const GemvArgs &a, int cu_count)
             return hipErrorInvalidValue;
         }
     }
-    return epi == EPI_ARGMAX || epi == EPI_QKV_ATTN ? hipErrorInvalidValue : launch_gemv_loop(st, epi, a, cu_count);
+    return epi == EPI_ARGMAX || epi == EPI_QKV_ATTN || epi == EPI_FFN ? hipErrorInvalidValue
+                                                                      : launch_gemv_loop(st, epi, a, cu_count);
 }
 
 // ---------------------------------------------------------------------------------------------------------------

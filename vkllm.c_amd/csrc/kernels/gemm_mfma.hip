@@ -46,14 +46,17 @@ __device__ __forceinline__ void gemm_store(int epi, uint16_t *C, uint32_t ldc, u
         *c = f2h(h2f(*c) + h2f(f2h(v)));
 }
 
-// GEMM_SWIGLU: product column c of [Wu; Wg] (F rows each, F % 32 == 0) is up row 32 (c / 64) + c % 32 when
-// (c / 32) is even, else gate row F + 32 (c / 64) + c % 32; the output column of up column c is 32 (c / 64) + c % 32
-template <int EPI> __device__ __forceinline__ uint32_t gemm_b_row(uint32_t c, uint32_t F)
+// products of interleaved up and gate columns
+__host__ __device__ constexpr bool is_dual(int epi)
 {
-    if constexpr (EPI == GEMM_SWIGLU)
-        return 32 * (c / 64) + c % 32 + ((c / 32) % 2) * F;
-    else
-        return c;
+    return epi == GEMM_SWIGLU || epi == GEMM_FFN;
+}
+
+// Dual products: product column c is up row 32 (c / 64) + c % 32 when (c / 32) is even, else the gate row of that
+// number; the output column of up column c is 32 (c / 64) + c % 32
+template <int EPI> __device__ __forceinline__ uint16_t dual_out(float up, float gate)
+{
+    return EPI == GEMM_FFN ? ffn_out(up, gate) : swiglu_out(up, gate);
 }
 __device__ __forceinline__ uint32_t swiglu_col(uint32_t c)
 {
@@ -238,11 +241,12 @@ __device__ __forceinline__ void for_seq(std::integer_sequence<int, J...>, F &&f)
 // register sets, 128 x 128 tiles only, one workgroup per CU for the registers) keeps the whole K of a short prompt's
 // tile in one workgroup.
 // n_base: product column of the kernel's column 0 (B rows and C columns are addressed from it; N counts the
-// kernel's columns). GEMM_SWIGLU reads the product's columns from [Wu; Wg] as interleaved 32-row blocks and
-// `split` holds F.
+// kernel's columns). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
+// blocks and `split` holds F.
 template <int BM, int BN, int EPI, bool SPLIT, int PF = 1>
 __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const uint16_t *__restrict__ A,
-                                                        const uint16_t *__restrict__ B, uint16_t *C, float *work,
+                                                        const uint16_t *__restrict__ B,
+                                                        const uint16_t *__restrict__ B2, uint16_t *C, float *work,
                                                         uint32_t M, uint32_t N, uint32_t K, uint32_t ldc,
                                                         uint32_t split, uint32_t kchunk, uint32_t tiles_m,
                                                         uint32_t tiles_total, uint32_t n_base, GemmRope rope)
@@ -281,8 +285,11 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
 #pragma unroll
     for (int i = 0; i < BV; ++i)
     {
+        // row v / 8 = tid / 8 + 32 i of the tile: for dual products of up and gate blocks in turn
         const uint32_t v = tid + 256 * i;
-        boff[i] = gemm_b_row<EPI>(n_base + min(n0 + v / 8, N - 1), split) * K + (v % 8) * 8;
+        const uint32_t row = is_dual(EPI) ? min((n_base + n0) / 2 + 32 * (i / 2) + tid / 8, split - 1)
+                                          : n_base + min(n0 + v / 8, N - 1);
+        boff[i] = row * K + (v % 8) * 8;
     }
     auto load = [&](auto set_tag, uint32_t k0) {
         constexpr int S = decltype(set_tag)::value;
@@ -294,7 +301,8 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
         }
 #pragma unroll
         for (int i = 0; i < BV; ++i)
-            rb[S][i] = __builtin_nontemporal_load((const u32x4 *)(B + boff[i] + k0));
+            rb[S][i] = __builtin_nontemporal_load(
+                (const u32x4 *)((is_dual(EPI) && i % 2 ? B2 : B) + boff[i] + k0));
     };
     auto stash = [&](auto set_tag, int buf) {
         constexpr int S = decltype(set_tag)::value;
@@ -474,7 +482,7 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
         // Epilogue through LDS (the K-step buffers are free now): each lane writes its fp16 outputs into a row-major
         // tile, then the workgroup moves 16-byte row chunks to their destinations, so the stores (and the residual's
         // loads) are whole vectors instead of one 2-byte element per lane. SwiGLU tiles have BN / 2 output columns.
-        constexpr int OC = EPI == GEMM_SWIGLU ? BN / 2 : BN;
+        constexpr int OC = is_dual(EPI) ? BN / 2 : BN;
         constexpr int TROW = OC + 8; // halves; rows 4 apart then start 16 banks apart
         static_assert(BM * TROW <= 2 * (BM + BN) * kLdsRow, "epilogue tile fits the K-step buffers");
         __syncthreads();
@@ -482,14 +490,14 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; j += (EPI == GEMM_SWIGLU ? 2 : 1))
+            for (int j = 0; j < TN; j += (is_dual(EPI) ? 2 : 1))
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
                 {
                     const uint32_t rt = wm * WM + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
                     const uint32_t ct = wn * WN + j * 32 + lane % 32;
-                    if constexpr (EPI == GEMM_SWIGLU)
-                        T[rt * TROW + swiglu_col(ct)] = swiglu_out(acc[i][j][e], acc[i][j + 1][e]);
+                    if constexpr (is_dual(EPI))
+                        T[rt * TROW + swiglu_col(ct)] = dual_out<EPI>(acc[i][j][e], acc[i][j + 1][e]);
                     else if constexpr (EPI == GEMM_SILU_HI)
                         T[rt * TROW + ct] = f2h(n_base + n0 + ct >= split ? silu(acc[i][j][e]) : acc[i][j][e]);
                     else
@@ -497,8 +505,9 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
                 }
         __syncthreads();
         constexpr int CH = OC / 8;
-        const uint32_t oc0 = EPI == GEMM_SWIGLU ? (n_base + n0) / 2 : n_base + n0; // output column of tile column 0
-        const uint32_t oce = EPI == GEMM_SWIGLU ? (n_base + N) / 2 : n_base + N;   // end of this launch's columns
+        const uint32_t oc0 = is_dual(EPI) ? (n_base + n0) / 2 : n_base + n0; // output column of tile column 0
+        // end of this launch's columns
+        const uint32_t oce = is_dual(EPI) ? min((n_base + N) / 2, split) : n_base + N;
         const bool vec = ((uintptr_t)C % 16 == 0) && ldc % 8 == 0;
         for (uint32_t idx = tid; idx < (uint32_t)(BM * CH); idx += 256)
         {
@@ -595,7 +604,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
         }
         return;
     }
-    if constexpr (EPI == GEMM_SWIGLU)
+    if constexpr (is_dual(EPI))
     {
         // 8 output columns f..f + 7 (inside one 32-column block): up columns c..c + 7, gate columns c + 32..c + 39
         const uint32_t per_row = N / 16;
@@ -603,13 +612,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
         for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < chunks; i += (uint64_t)gridDim.x * 256)
         {
             const uint32_t m = (uint32_t)(i / per_row), f = 8 * (uint32_t)(i % per_row), c = 64 * (f / 32) + f % 32;
+            if (n_base / 2 + f >= split) // columns past F (GEMM_FFN with F % 32 != 0)
+                continue;
             float up[8], gate[8];
             sum8((size_t)m * N + c, up);
             sum8((size_t)m * N + c + 32, gate);
             u32x4 o;
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                o[k] = pack2(swiglu_out(up[2 * k], gate[2 * k]), swiglu_out(up[2 * k + 1], gate[2 * k + 1]));
+                o[k] = pack2(dual_out<EPI>(up[2 * k], gate[2 * k]), dual_out<EPI>(up[2 * k + 1], gate[2 * k + 1]));
             *(u32x4 *)(C + (size_t)m * ldc + swiglu_col(n_base + c)) = o;
         }
         return;
@@ -663,7 +674,7 @@ template <int EPI>
 static uint32_t reduce_grid(uint32_t M, uint32_t N, uint32_t ldc, uint32_t n_base, const uint16_t *C)
 {
     uint64_t items = (uint64_t)M * N;
-    if (EPI == GEMM_SWIGLU)
+    if (is_dual(EPI))
         items /= 16;
     else if (EPI == GEMM_QKV_ROPE || reduce_vec8(N, ldc, n_base, C))
         items /= 8;
@@ -809,6 +820,12 @@ static hipError_t launch_resid_norm(hipStream_t st, const float *work, uint16_t 
     return hipGetLastError();
 }
 
+// the weight rows: p2 the gate rows of a dual product, whose up rows are p
+struct GemmB
+{
+    const uint16_t *p, *p2;
+};
+
 template <int BM, int BN> static size_t gemm_lds()
 {
     return (size_t)2 * (BM + BN) * kLdsRow * sizeof(uint16_t);
@@ -832,7 +849,7 @@ static hipError_t launch_tile(hipStream_t st, const uint16_t *A, const uint16_t 
 }
 
 template <int BM, int BN, int EPI, bool SPLIT, int PF = 1>
-static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, const uint16_t *B, uint16_t *C, float *work,
+static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                 uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
                                 uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
 {
@@ -844,7 +861,7 @@ static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, const uint16_
     const uint32_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, total = tm * tn;
     const uint32_t grid = (total + 7) / 8 * 8;
     gemm32_kernel<BM, BN, EPI, SPLIT, PF><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
-        A, B, C, work, M, N, K, ldc, split, kchunk, tm, total, n_base, rope ? *rope : GemmRope{});
+        A, B.p, B.p2, C, work, M, N, K, ldc, split, kchunk, tm, total, n_base, rope ? *rope : GemmRope{});
     return hipGetLastError();
 }
 
@@ -859,7 +876,7 @@ static hipError_t launch_reduce(hipStream_t st, const float *work, uint16_t *C, 
 }
 
 template <int BM, int BN, int EPI>
-static hipError_t launch_shape32(hipStream_t st, const uint16_t *A, const uint16_t *B, uint16_t *C, float *work,
+static hipError_t launch_shape32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                  uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
                                  uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
 {
@@ -890,7 +907,7 @@ static hipError_t launch_shape(hipStream_t st, const uint16_t *A, const uint16_t
 }
 
 template <int EPI>
-static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, const uint16_t *B, uint16_t *C, float *work,
+static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                   size_t work_elems, uint32_t M, uint32_t N, uint32_t K, uint32_t ldc,
                                   uint32_t split, int cu_count, const GemmRope *rope, const GemmNorm *norm,
                                   bool *normed)
@@ -902,8 +919,9 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, const uint1
             return hipErrorInvalidValue;
     if ((uint64_t)N * K >= (1ull << 32)) // B row offsets are 32-bit
         return hipErrorInvalidValue;
-    if constexpr (EPI == GEMM_SWIGLU)
-        if (K % kBK != 0 || N % 64 != 0 || N != 2 * split || ldc % 8 != 0 || (uintptr_t)C % 16 != 0)
+    if constexpr (is_dual(EPI))
+        if (K % kBK != 0 || N % 64 != 0 || N != (2 * split + 63) / 64 * 64 || split % 8 != 0 || !B.p2 || ldc % 8 != 0 ||
+            (uintptr_t)C % 16 != 0)
             return hipErrorInvalidValue;
     if (K % kBK == 0)
     {
@@ -1005,7 +1023,7 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, const uint1
             }
         return launch_shape32<128, 128, EPI>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, 0, rope);
     }
-    if constexpr (EPI == GEMM_SWIGLU || EPI == GEMM_QKV_ROPE)
+    if constexpr (is_dual(EPI) || EPI == GEMM_QKV_ROPE)
         return hipErrorInvalidValue; // checked above: not reached
     else
     {
@@ -1019,12 +1037,12 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, const uint1
                 splits *= 2;
             const uint32_t kchunk = ((K + splits - 1) / splits + kBK - 1) / kBK * kBK;
             splits = (K + kchunk - 1) / kchunk;
-            return launch_shape<128, 64, EPI>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk);
+            return launch_shape<128, 64, EPI>(st, A, B.p, C, work, M, N, K, ldc, split, splits, kchunk);
         }
         const uint64_t big = (uint64_t)((M + 127) / 128) * ((N + 127) / 128);
         if (big >= cus)
-            return launch_shape<128, 128, EPI>(st, A, B, C, work, M, N, K, ldc, split, 1, K);
-        return launch_shape<128, 64, EPI>(st, A, B, C, work, M, N, K, ldc, split, 1, K);
+            return launch_shape<128, 128, EPI>(st, A, B.p, C, work, M, N, K, ldc, split, 1, K);
+        return launch_shape<128, 64, EPI>(st, A, B.p, C, work, M, N, K, ldc, split, 1, K);
     }
 }
 
@@ -1052,34 +1070,39 @@ hipError_t launch_gemm_reduce(hipStream_t st, int epi, const float *work, uint16
 
 hipError_t launch_gemm(hipStream_t st, int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, uint32_t M,
                        uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, int cu_count, float *work,
-                       size_t work_elems, const GemmRope *rope, const GemmNorm *norm)
+                       size_t work_elems, const GemmRope *rope, const GemmNorm *norm, const uint16_t *B2)
 {
     if (K % 8 != 0 || K < 8 || M == 0 || N == 0)
         return hipErrorInvalidValue;
     switch (epi)
     {
     case GEMM_PLAIN:
-        return launch_epi_gemm<GEMM_PLAIN>(st, A, B, C, work, work_elems, M, N, K, ldc, split, cu_count, nullptr,
+        return launch_epi_gemm<GEMM_PLAIN>(st, A, GemmB{B, nullptr}, C, work, work_elems, M, N, K, ldc, split, cu_count, nullptr,
                                              nullptr, nullptr);
     case GEMM_SILU_HI:
-        return launch_epi_gemm<GEMM_SILU_HI>(st, A, B, C, work, work_elems, M, N, K, ldc, split, cu_count, nullptr,
+        return launch_epi_gemm<GEMM_SILU_HI>(st, A, GemmB{B, nullptr}, C, work, work_elems, M, N, K, ldc, split, cu_count, nullptr,
                                              nullptr, nullptr);
     case GEMM_RESID:
     {
         if (norm && (ldc != N || N % 8 != 0))
             return hipErrorInvalidValue;
         bool normed = false;
-        hipError_t e = launch_epi_gemm<GEMM_RESID>(st, A, B, C, work, work_elems, M, N, K, ldc, split, cu_count,
+        hipError_t e = launch_epi_gemm<GEMM_RESID>(st, A, GemmB{B, nullptr}, C, work, work_elems, M, N, K, ldc, split, cu_count,
                                                    nullptr, norm, &normed);
         if (e != hipSuccess || !norm || normed)
             return e;
         return launch_rmsnorm_rows(st, C, norm->w, norm->y, M, N, norm->eps, norm->xt);
     }
     case GEMM_SWIGLU:
-        return launch_epi_gemm<GEMM_SWIGLU>(st, A, B, C, work, work_elems, M, N, K, ldc, split, cu_count, nullptr,
-                                             nullptr, nullptr);
+        if (N != 2 * split)
+            return hipErrorInvalidValue;
+        return launch_epi_gemm<GEMM_SWIGLU>(st, A, GemmB{B, B + (size_t)split * K}, C, work, work_elems, M, N, K, ldc,
+                                            split, cu_count, nullptr, nullptr, nullptr);
+    case GEMM_FFN:
+        return launch_epi_gemm<GEMM_FFN>(st, A, GemmB{B, B2}, C, work, work_elems, M, N, K, ldc, split, cu_count,
+                                         nullptr, nullptr, nullptr);
     case GEMM_QKV_ROPE:
-        return launch_epi_gemm<GEMM_QKV_ROPE>(st, A, B, C, work, work_elems, M, N, K, ldc, split, cu_count, rope,
+        return launch_epi_gemm<GEMM_QKV_ROPE>(st, A, GemmB{B, nullptr}, C, work, work_elems, M, N, K, ldc, split, cu_count, rope,
                                               nullptr, nullptr);
     default:
         return hipErrorInvalidValue;

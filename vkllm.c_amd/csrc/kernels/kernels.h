@@ -84,6 +84,9 @@ enum GemvEpi : int
     // workgroup that completes the head's q, k and v rows: attn_out[h*hd + d] as the short-cache attention kernel
     // leaves it. head_count [H] counts completed units per head (zero between launches).
     EPI_QKV_ATTN = 6,
+    // the FFN_UP_AND_GATE op's single row: w holds the up rows, w2 the gate rows (`rows` of each), the input as given:
+    // out[r] = fp16(up_r * gate_r / (1 + exp(-gate_r))), rounded once
+    EPI_FFN = 7,
 };
 // the decode QKV product's attention tail: heads at most, and positions at most (its scores and partial sums reuse
 // the GEMV's input LDS, sized to hold kAttnTailMaxKv + 4 * hd floats)
@@ -95,6 +98,7 @@ struct GemvArgs
     const float *norm_w;    // RMSNorm weight: x is normalised in the prologue; nullptr: x used as is
     float eps;
     const uint16_t *w;      // weight rows [rows, K], K contiguous
+    const uint16_t *w2;     // EPI_FFN: the gate rows [rows, K]
     uint32_t K;
     uint32_t units;         // fallback kernel (K > 14336) work units: PLAIN/RESID ceil(rows/2), GATEUP F, QKV 3D/2
     uint32_t rows_per_unit; // rows a wave reduces at once (1, 2 or 4); 0 picks the default for the shape
@@ -258,6 +262,9 @@ enum GemmEpi : int
     // as the prompt step's q, k and v: q and k rotated by RoPE (each element first rounded to fp16, then the
     // rotation of launch_rope_kv), q -> rope.q[m][c], k and v -> the caches at that position; C is not written
     GEMM_QKV_ROPE = 4,
+    // GEMM_SWIGLU's product with up rows B and gate rows B2 in matrices of their own (F = split rows each, F % 8 == 0,
+    // N = 2 F rounded up to a multiple of 64), as the FFN_UP_AND_GATE op rounds it: once, from the fp32 sums
+    GEMM_FFN = 5,
 };
 struct GemmRope
 {
@@ -277,11 +284,12 @@ struct GemmNorm
 };
 // C[M, N] (row stride ldc) = A[M, K] . B[N, K]^T, fp16 operands, fp32 accumulation on MFMA. K % 8 == 0.
 // `work` (work_elems floats) holds split-K partial tiles for short prompts; with too little of it K is not split.
-// `rope` is read by GEMM_QKV_ROPE only; `norm` (GEMM_RESID only) adds the RMSNorm of the updated rows, fused into
+// `rope` is read by GEMM_QKV_ROPE only, B2 by GEMM_FFN only; `norm` (GEMM_RESID only) adds the RMSNorm of the updated rows, fused into
 // the split-K reduce when K is split.
 hipError_t launch_gemm(hipStream_t st, int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, uint32_t M,
                        uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, int cu_count, float *work,
-                       size_t work_elems, const GemmRope *rope = nullptr, const GemmNorm *norm = nullptr);
+                       size_t work_elems, const GemmRope *rope = nullptr, const GemmNorm *norm = nullptr,
+                       const uint16_t *B2 = nullptr);
 // Prompt-step products of at most 128 tokens with the weights read from a fragment-tiled copy (launch_tile_weights)
 // and X fragment-ordered (xt_vec): C[M, N] = X[M, K] . W[N, K]^T, M <= 128, K % 16 == 0.
 enum StreamEpi : int
