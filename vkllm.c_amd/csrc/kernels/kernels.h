@@ -31,6 +31,10 @@ hipError_t launch_rmsnorm(hipStream_t st, const TView &x, const TView &w, const 
 // out = act(scale * a . b), b [N,K] when transposed_b else [K,N]; size-1 batch dims broadcast
 hipError_t launch_matmul(hipStream_t st, const TView &a, const TView &b, const TView &out, float scale, int act,
                          bool transposed_b);
+// the same on matrix cores for fp16 views of contiguous rows (s[3] == 1; any alignment, other strides and batches)
+bool matmul_batched_ok(const TView &a, const TView &b, const TView &out);
+hipError_t launch_matmul_batched(hipStream_t st, const TView &a, const TView &b, const TView &out, float scale, int act,
+                                 bool transposed_b, int cu_count);
 // freqs_host[w] = base^(2w/D) for w < D/2 (D <= 2*kMaxRopeFreqs), passed by value in the kernel arguments
 constexpr int kMaxRopeFreqs = 256;
 hipError_t launch_rope(hipStream_t st, const TView &in, const TView &out, uint32_t offset, const float *freqs_host,

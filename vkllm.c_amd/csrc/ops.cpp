@@ -277,13 +277,16 @@ static bool is_mat_mul_vec(const vkllm_tensor *t)
 // fp16 A [1,1,M,K], B [1,1,N,K] (is_transposed_b) and out [1,1,M,N], rows contiguous, K a multiple of 8, 16-byte
 // aligned rows, scale 1. M == 1 (the reference's mat_mul_vec case) takes the streaming GEMV (16-byte weight loads,
 // fp32 accumulation, DPP wave sums) when act is 0; M > 1 takes the MFMA tile GEMM, act 1 as its SiLU epilogue.
-// Anything else (fp32, broadcast batches, B as [K, N], a scale, strided views) runs the generic kernels. Both keep
-// the reference's rounding points (fp32 sums, then fp16(act(scale * acc))), so only the fp32 summation order differs.
+// Other fp16 products of contiguous rows (batches, B as [K, N], a scale, ragged or strided rows) run on the batched
+// matrix-core kernel, but for the reference's mat_mul_vec case, which streams B once from a wave per result. Anything
+// else (fp32, rows that are not contiguous) runs the generic kernels. All keep the reference's rounding points (fp32
+// sums, then fp16(act(scale * acc))), so only the fp32 summation order differs.
 enum MatmulPath
 {
     GENERIC,
     FAST_GEMV,
-    FAST_GEMM
+    FAST_GEMM,
+    BATCHED
 };
 
 static bool rows_fp16(const vk::TView &v, uint32_t rows, uint32_t cols)
@@ -296,12 +299,13 @@ static MatmulPath matmul_fast_path(const vk::TView &a, const vk::TView &b, const
                                    const vkllm_op_matmul_params &p, bool transposed_b)
 {
     const uint32_t M = out.n[2], N = out.n[3], K = a.n[3];
+    const MatmulPath other = !(M == 1 && transposed_b) && vk::matmul_batched_ok(a, b, out) ? BATCHED : GENERIC;
     if (!transposed_b || p.scale != 1.0f || K % 8 != 0 || !rows_fp16(a, M, K) || !rows_fp16(b, N, K) ||
         !rows_fp16(out, M, N) || (M > 1 && a.s[2] != K) || b.s[2] != K)
-        return GENERIC;
+        return other;
     if (M == 1)
         return p.act == 0 ? FAST_GEMV : GENERIC;
-    return p.act == 0 || p.act == 1 ? FAST_GEMM : GENERIC;
+    return p.act == 0 || p.act == 1 ? FAST_GEMM : other;
 }
 
 static hipError_t launch_op_gemv(vkllm_context *ctx, const vk::TView &a, const vk::TView &b, const vk::TView &out)
@@ -403,6 +407,11 @@ extern "C" vkllm_err_t vkllm_op_matmul_run(struct vkllm_context *context, struct
                                context->device->cu_count, work, work_elems));
         break;
     }
+    case BATCHED:
+        LAUNCH(context, kid,
+               vk::launch_matmul_batched(context->device->stream, av, bv, out, p.scale, p.act, tb,
+                                         context->device->cu_count));
+        break;
     default:
         LAUNCH(context, kid, vk::launch_matmul(context->device->stream, av, bv, out, p.scale, p.act, tb));
     }
