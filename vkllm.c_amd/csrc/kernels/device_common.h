@@ -198,6 +198,20 @@ __device__ __forceinline__ float half_hi(uint32_t v)
     return h2f((uint16_t)(v >> 16));
 }
 
+// 8 halfs at an address of any parity: global memory takes unaligned 16-byte accesses
+struct __attribute__((packed, aligned(2))) Half8
+{
+    u32x4 v;
+};
+__device__ __forceinline__ u32x4 load_half8(const uint16_t *p)
+{
+    return ((const Half8 *)p)->v;
+}
+__device__ __forceinline__ void store_half8(uint16_t *p, u32x4 v)
+{
+    ((Half8 *)p)->v = v;
+}
+
 // 8-element fp16 dot product accumulated in fp32 (fp16 -> fp32 widening FMAs, v_fma_mix_f32). The
 // v_dot2_f32_f16 builtin gave wrong sums on gfx950 and is not used.
 __device__ __forceinline__ float dot8(u32x4 w, u32x4 x, float acc)

