@@ -2,15 +2,11 @@
 // It replaces src/shaders/vkllm_matmul_t1.comp for the token step's weight products, where A holds the step's
 // activations (M = tokens) and B a weight matrix stored [out, in].
 //
-// gemm32_kernel (K a multiple of 64, every prefill product of the LLaMA-2 shapes): v_mfma_f32_32x32x16_f16 on
-// 256 x 256 or 128 x 128 tiles of 256-thread workgroups, 2 x 2 waves each owning a (BM/2) x (BN/2) grid of 32x32
-// blocks (up to 256 fp32 accumulators per lane), K in steps of 64 through two LDS buffers with rows padded to 144
-// bytes (the operand reads of 8 lanes then fall on distinct banks). A step is straight-line code whose instruction
-// stream group barriers lay out as MFMAs with, between them, the next 16-wide slice's operand reads, the next
-// step's global loads (first slice) and their stores into the other LDS buffer (last slice), so memory traffic
-// runs under the matrix pipe; one barrier per step. Its epilogue stages the tile's fp16 outputs in the freed LDS and
-// stores 16-byte row chunks: plain, SiLU on columns >= split, residual add, the FFN's SwiGLU (reading [Wu; Wg] as
-// interleaved 32-row blocks), or the QKV product's RoPE with q and the K/V cache rows written directly.
+// gemm32_kernel (K a multiple of 64, every prefill product of the LLaMA-2 shapes): v_mfma_f32_32x32x16_f16 on tiles of 64
+// x 128 to 256 x 256 by 256-thread workgroups, operands copied straight into a ring of LDS buffers, one barrier per 64 of
+// K (described at the kernel). Its epilogue stages the tile's fp16 outputs in the freed LDS and stores 16-byte row chunks:
+// plain, SiLU on columns >= split, residual add, the FFN's up * silu(gate) (reading up and gate rows as interleaved
+// 16-row blocks), or the QKV product's RoPE with q and the K/V cache rows written directly.
 // gemm_kernel (other K): v_mfma_f32_16x16x32_f16, 128 x 128 or 128 x 64 tiles, the same double buffering, with the
 // K tail zeroed (plain, SiLU and residual epilogues only).
 //
@@ -19,6 +15,9 @@
 // gemm_resid_norm_kernel, which also normalises the rows. Tiles are ordered M-fastest and dealt to XCDs in
 // contiguous runs so a run shares its B tiles in one L2. Global loads are unconditional at clamped addresses (a
 // guarded load compiles to a branch and a wait per load).
+#include <float.h>
+
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -52,56 +51,57 @@ __host__ __device__ constexpr bool is_dual(int epi)
     return epi == GEMM_SWIGLU || epi == GEMM_FFN;
 }
 
-// Dual products: product column c is up row 32 (c / 64) + c % 32 when (c / 32) is even, else the gate row of that
-// number; the output column of up column c is 32 (c / 64) + c % 32
+// Dual products: product column c is up row 16 (c / 32) + c % 16 when (c / 16) is even, else the gate row of that
+// number, so both values of an output lie in one 32-column MFMA block, 16 lanes apart; the output column of up column c
+// is 16 (c / 32) + c % 16
 template <int EPI> __device__ __forceinline__ uint16_t dual_out(float up, float gate)
 {
     return EPI == GEMM_FFN ? ffn_out(up, gate) : swiglu_out(up, gate);
 }
 __device__ __forceinline__ uint32_t swiglu_col(uint32_t c)
 {
-    return 32 * (c / 64) + c % 32;
-}
-
-// GEMM_QKV_ROPE: element (m, c) of region `region` (0 q, 1 k, 2 v) at head `head`, head dim `dim`; v is the
-// element's fp16-rounded value and w its RoPE partner's (dim ^ 1), as launch_rope_kv combines them
-__device__ __forceinline__ void rope_store(const GemmRope &r, uint32_t m, uint32_t region, uint32_t c,
-                                           uint32_t head, uint32_t dim, float v, float w)
-{
-    const size_t cache = ((size_t)head * r.ctx + r.offset + m) * r.hd + dim;
-    if (region == 2)
-    {
-        r.vc[cache] = f2h(v);
-        return;
-    }
-    const float *cs = r.cs + ((size_t)m * (r.hd / 2) + dim / 2) * 2;
-    const float out = (dim & 1) == 0 ? rope_mul_sub(cs[0], v, cs[1], w) : rope_mul_add(cs[1], w, cs[0], v);
-    if (region == 0)
-        r.q[(size_t)m * r.D + c] = f2h(out);
-    else
-        r.kc[cache] = f2h(out);
+    return 16 * (c / 32) + c % 16;
 }
 
 // GEMM_QKV_ROPE: 8 consecutive product columns from `a` (a multiple of 8) of row m, as fp16: four RoPE pairs of q
-// or k rotated and stored, or v stored, as one 16-byte vector each
-__device__ __forceinline__ void rope_store8(const GemmRope &r, uint32_t m, uint32_t a, u32x4 v)
+// or k rotated and stored, or v stored, as one 16-byte vector each. rope_load8 fetches the pairs' (cos, sin).
+struct Rope8
 {
-    const uint32_t region = (a >= r.D) + (a >= 2 * r.D), c = a - region * r.D, head = c / r.hd, dim = c % r.hd;
+    float4 lo, hi;
+};
+__device__ __forceinline__ Rope8 rope_load8(const GemmRope &r, uint32_t m, uint32_t a)
+{
+    const uint32_t region = (a >= r.D) + (a >= 2 * r.D), dim = (a - region * r.D) & (r.hd - 1); // hd: a power of two
+    const float4 *cs = (const float4 *)(r.cs + (size_t)m * r.hd + dim);
+    return {cs[0], cs[1]};
+}
+__device__ __forceinline__ void rope_store8(const GemmRope &r, uint32_t m, uint32_t a, u32x4 v, const Rope8 &cs)
+{
+    const uint32_t region = (a >= r.D) + (a >= 2 * r.D), c = a - region * r.D;
+    const uint32_t head = c >> (31 - __clz((int)r.hd)), dim = c & (r.hd - 1);
     const size_t cache = ((size_t)head * r.ctx + r.offset + m) * r.hd + dim;
     if (region == 2)
     {
         *(u32x4 *)(r.vc + cache) = v;
         return;
     }
-    const float *cs = r.cs + ((size_t)m * (r.hd / 2) + dim / 2) * 2;
+    const float f[8] = {cs.lo.x, cs.lo.y, cs.lo.z, cs.lo.w, cs.hi.x, cs.hi.y, cs.hi.z, cs.hi.w};
     u32x4 o;
 #pragma unroll
     for (int k = 0; k < 4; ++k)
     {
-        const float x0 = half_lo(v[k]), x1 = half_hi(v[k]), co = cs[2 * k], sn = cs[2 * k + 1];
+        const float x0 = half_lo(v[k]), x1 = half_hi(v[k]), co = f[2 * k], sn = f[2 * k + 1];
         o[k] = pack2(f2h(rope_mul_sub(co, x0, sn, x1)), f2h(rope_mul_add(sn, x0, co, x1)));
     }
     *(u32x4 *)(region == 0 ? r.q + (size_t)m * r.D + c : r.kc + cache) = o;
+}
+// fp16(r + v) of 8 columns
+__device__ __forceinline__ u32x4 resid8(u32x4 r, u32x4 v)
+{
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        v[k] = pack2(f2h(half_lo(r[k]) + half_lo(v[k])), f2h(half_hi(r[k]) + half_hi(v[k])));
+    return v;
 }
 
 // SPLIT: workgroup z of gridDim.y covers K columns [z * kchunk, min(K, (z + 1) * kchunk)) and writes its fp32 tile
@@ -221,41 +221,62 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint16_t *__restrict__ 
             }
 }
 
-// The same product on v_mfma_f32_32x32x16_f16 with larger wave tiles: 4 waves as 2 x 2 of (BM/2) x (BN/2), each a
-// grid of 32x32 MFMA blocks (up to 4 x 4: 256 fp32 accumulators per lane). A wave tile of 128 x 128 reads half the
-// LDS bytes per flop of a 64 x 64 one. Operands: lane l holds row (l % 32) of a 32-row block at K offset
-// 8 (l / 32) of each 16-wide K slice; the block's accumulator element e of lane l is C[8 (e / 4) + 4 (l / 32) +
-// e % 4][l % 32]. Loads, LDS layout, tile order and split-K as in gemm_kernel.
+// The same product on v_mfma_f32_32x32x16_f16, pipelined by hand: 4 waves as 2 x 2 of (BM/2) x (BN/2), each a grid of
+// 32x32 MFMA blocks (up to 4 x 4: 256 fp32 accumulators per lane, so one wave per SIMD and nothing else to hide
+// latency behind). Operands: lane l holds row (l % 32) of a 32-row block at K offset 8 (l / 32) of each 16-wide K slice;
+// the block's accumulator element e of lane l is C[8 (e / 4) + 4 (l / 32) + e % 4][l % 32].
+//
+// Memory side. global_load_lds copies the operands into LDS without passing registers, 8 rows of 128 bytes (64 of K:
+// whole cache lines) per instruction; the 16-byte chunks of a row are placed XORed by the row's low bits, which makes
+// the operand reads of 8 lanes fall on distinct banks without padding the copies could not write. 64 of K arrive as two
+// halves, half h being the rows of the waves with wm == h and wn == h, through a ring of NH halves (5 of 32 KB for
+// 256 x 256 tiles: all of a CU's LDS). In step s (32 of K) every wave issues its share of half s + NH - 1.
+//
+// Compute side. A step's MFMAs run on operands read from LDS one step earlier (two register sets of two 16-wide slices),
+// so neither LDS latency nor the barrier's skew reaches the matrix pipe; the next step's operand reads and the copies
+// are threaded between the MFMAs, in the order written (sched_barrier pins it). Only every second step ends in a wait
+// for copies and a barrier: a half's slot is written again no earlier than the step after the barrier that follows its
+// last read, and before that barrier each wave has waited for its own copies of the two halves read next.
+// The copies are written in assembly because the compiler would put a wait for all of them before every LDS read; they
+// have no register results, and the waits for them are the ones written here.
+//
+// What bounds it: L2 to LDS copies at ~68 bytes/ns of a CU for tiles below 256 x 256, and for whole-chip products the
+// matrix pipes at the clock the chip sustains (with copies and LDS reads switched off a 2048 x 15360 x 5120 product
+// takes 219 us, without the copies 232, whole 271). Before (operands staged through registers, 144-byte LDS rows, one
+// wait per slice) and now, us: 1024 x 12288 x 4096 127 / 92 (1.11 PFLOP/s), 2048 x 15360 x 5120 323 / 271-298,
+// 2048 x 5120 x 13824 346 / 257, 1024 x 4096 x 4096 47 / 36, 301 x 12288 x 4096 74 / 46.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // f(integral_constant<int, J>) for J in the sequence, in order
 template <int... J, typename F>
-__device__ __forceinline__ void for_seq(std::integer_sequence<int, J...>, F &&f)
+__host__ __device__ __forceinline__ void for_seq(std::integer_sequence<int, J...>, F &&f)
 {
     (f(std::integral_constant<int, J>{}), ...);
 }
 
-// PF: K steps whose global loads are in flight at once. With PF 2 the loads run two steps ahead through two register
-// sets (a step's loads are stored to LDS at the end of the following step); a split tile of a short prompt has little
-// MFMA work per step, and one step of loads in flight leaves it waiting on memory latency every step. PF 4 (four
-// register sets, 128 x 128 tiles only, one workgroup per CU for the registers) keeps the whole K of a short prompt's
-// tile in one workgroup.
+// halves in the LDS ring: as many as fit 160 KB, up to 10
+template <int BM, int BN> constexpr int gemm_ring()
+{
+    constexpr int fit = 160 * 1024 / ((BM + BN) * 64);
+    return fit < 10 ? fit : 10;
+}
+
 // n_base: product column of the kernel's column 0 (B rows and C columns are addressed from it; N counts the
 // kernel's columns). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
 // blocks and `split` holds F.
-template <int BM, int BN, int EPI, bool SPLIT, int PF = 1>
-__global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const uint16_t *__restrict__ A,
-                                                        const uint16_t *__restrict__ B,
+template <int BM, int BN, int EPI, bool SPLIT>
+__global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                         const uint16_t *__restrict__ B2, uint16_t *C, float *work,
                                                         uint32_t M, uint32_t N, uint32_t K, uint32_t ldc,
                                                         uint32_t split, uint32_t kchunk, uint32_t tiles_m,
                                                         uint32_t tiles_total, uint32_t n_base, GemmRope rope)
 {
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int AV = BM * kBK / 8 / 256, BV = BN * kBK / 8 / 256; // 16-byte vectors per thread per K step
-    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-    auto As = [&](int b) { return lds + b * BM * kLdsRow; };
-    auto Bs = [&](int b) { return lds + 2 * BM * kLdsRow + b * BN * kLdsRow; };
+    constexpr int HALF = (BM + BN) * 64, NH = gemm_ring<BM, BN>(); // bytes of a half, halves in the ring
+    constexpr int ND = (BM + BN) / 64, NAI = WM / 32; // copies of a wave per half, the first NAI of them rows of A
+    constexpr int NR = 2 * (TM + TN), NM = 2 * TM * TN; // operand reads and MFMAs of a step
+    static_assert(WM % 32 == 0 && WN % 32 == 0 && NH >= 5, "whole MFMA blocks, and the waits below");
+    extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
 
     const uint32_t per_xcd = gridDim.x / 8;
     const uint32_t t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
@@ -264,8 +285,39 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
     const uint32_t m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
     const uint32_t kb = SPLIT ? blockIdx.y * kchunk : 0;
     const uint32_t ke = SPLIT ? min(K, kb + kchunk) : K;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wid >> 1, wn = wid & 1;
+
+    // Copy i of a wave and half h fills the half's LDS rows 8 (wid + 4 i) .. + 7 (WM rows of A, then WN of B), lane l
+    // row l / 8, chunk position l % 8. Rows past M or N repeat the last one: they only feed outputs that are not
+    // stored. Every K step lies wholly inside [kb, ke) (the launcher admits whole 64-wide steps).
+    const uint32_t n_first = is_dual(EPI) ? (n_base + n0) / 2 : n_base + n0; // first row of B (and B2)
+    const uint32_t n_last = is_dual(EPI) ? split - 1 : n_base + N - 1;
+    const char *const Ap = (const char *)(A + (size_t)m0 * K + kb);
+    // dual products: waves 0 and 1 copy the up rows of each block, waves 2 and 3 its gate rows
+    const char *const Bp = (const char *)((is_dual(EPI) && wid >= 2 ? B2 : B) + (size_t)n_first * K + kb);
+    uint32_t voff[2][ND]; // byte offsets from those
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+        {
+            const uint32_t r = 8 * wid + lane / 8; // the row in its block of 32
+            const int blk = i < NAI ? i + h * TM : i - NAI + h * TN;
+            const uint32_t row = i < NAI ? min(32 * blk + r, M - 1 - m0)
+                                         : min(is_dual(EPI) ? 16 * blk + r % 16 : 32 * blk + r, n_last - n_first);
+            voff[h][i] = row * K * 2 + ((lane ^ (r & 7)) & 7) * 16;
+        }
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)lds + wid * 1024;
+    auto copy = [&](auto h_tag, int i, uint32_t slot, uint32_t kbyte) {
+        constexpr int H = decltype(h_tag)::value;
+        const char *base = (i < NAI ? Ap : Bp) + kbyte;
+        const uint32_t to = lds_base + slot + i * 4096, off = voff[H][i];
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base)
+                     : "m0");
+    };
+    const uint32_t nsteps = (ke - kb) / 32, last_k = (nsteps / 2 - 1) * 128;
+    auto kat = [&](uint32_t half) { return min(half / 2 * 128, last_k); }; // halves past the end repeat the last K
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -276,228 +328,106 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
             for (int e = 0; e < 16; ++e)
                 acc[i][j][e] = 0.f;
 
-    // every K step lies wholly inside [kb, ke) (the launcher admits K ranges of whole 64-wide steps), so the
-    // loads need no masks and each step's body is straight-line code for the scheduler
-    u32x4 ra[PF][AV], rb[PF][BV];
-    // element offsets of this thread's B rows (fixed for the tile) at its 16-byte column of a K step; B has fewer
-    // than 2^32 elements (checked by the launcher)
-    uint32_t boff[BV];
-#pragma unroll
-    for (int i = 0; i < BV; ++i)
-    {
-        // row v / 8 = tid / 8 + 32 i of the tile: for dual products of up and gate blocks in turn
-        const uint32_t v = tid + 256 * i;
-        const uint32_t row = is_dual(EPI) ? min((n_base + n0) / 2 + 32 * (i / 2) + tid / 8, split - 1)
-                                          : n_base + min(n0 + v / 8, N - 1);
-        boff[i] = row * K + (v % 8) * 8;
-    }
-    auto load = [&](auto set_tag, uint32_t k0) {
+    f16x8 fr[2][2][TM + TN]; // [register set][slice]: A blocks, then B blocks
+    const uint32_t rl = lane % 32, at = rl * 128 + (((lane / 32) ^ (rl & 7)) * 16);
+    uint32_t slot_a = wm * HALF, slot_b = wn * HALF + WM * 128; // this wave's rows of the 64 of K being read
+    // operand x of slice sl of the step with K offset 32 p in its 64
+    auto read = [&](auto set_tag, int sl, int x, int p) {
         constexpr int S = decltype(set_tag)::value;
+        const uint32_t o = at ^ (64 * p + 32 * sl);
+        const char *q = (const char *)lds + (x < TM ? slot_a + o + x * 4096 : slot_b + o + (x - TM) * 4096);
+        fr[S][sl][x] = *(const f16x8 *)q;
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    // One step: the MFMAs of register set S, the reads of the next step (K offset 32 P) into the other set, and this
+    // wave's copies of a half with parity H into `slot`
+    auto step = [&](auto s_tag, auto p_tag, auto h_tag, uint32_t slot, uint32_t kbyte) {
+        constexpr int S = decltype(s_tag)::value;
+        using Other = std::integral_constant<int, 1 - S>;
+        int nr = 0, nd = 0;
 #pragma unroll
-        for (int i = 0; i < AV; ++i)
+        for (int k = 0; k < NM; ++k)
         {
-            const uint32_t v = tid + 256 * i, row = min(m0 + v / 8, M - 1);
-            ra[S][i] = *(const u32x4 *)(A + (size_t)row * K + k0 + (v % 8) * 8);
+            const int sl = k / (TM * TN), i = k % (TM * TN) / TN, j = k % TN;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[S][sl][i], fr[S][sl][TM + j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            // all issued by 7/8 of the step
+            const int want_r = min(NR, (k + 1) * NR * 8 / (NM * 7)), want_d = min(ND, (k + 1) * ND * 8 / (NM * 7));
+#pragma unroll
+            for (; nr < want_r; ++nr)
+                read(Other{}, nr / (TM + TN), nr % (TM + TN), decltype(p_tag)::value);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (; nd < want_d; ++nd)
+                copy(h_tag, nd, slot, kbyte);
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int i = 0; i < BV; ++i)
-            rb[S][i] = __builtin_nontemporal_load(
-                (const u32x4 *)((is_dual(EPI) && i % 2 ? B2 : B) + boff[i] + k0));
+        for (; nr < NR; ++nr)
+            read(Other{}, nr / (TM + TN), nr % (TM + TN), decltype(p_tag)::value);
+#pragma unroll
+        for (; nd < ND; ++nd)
+            copy(h_tag, nd, slot, kbyte);
     };
-    auto stash = [&](auto set_tag, int buf) {
-        constexpr int S = decltype(set_tag)::value;
-#pragma unroll
-        for (int i = 0; i < AV; ++i)
-        {
-            const uint32_t v = tid + 256 * i;
-            *(u32x4 *)(As(buf) + (v / 8) * kLdsRow + (v % 8) * 8) = ra[S][i];
-        }
-#pragma unroll
-        for (int i = 0; i < BV; ++i)
-        {
-            const uint32_t v = tid + 256 * i;
-            *(u32x4 *)(Bs(buf) + (v / 8) * kLdsRow + (v % 8) * 8) = rb[S][i];
-        }
-    };
-    f16x8 af[2][TM], bf[2][TN];
-    auto frags = [&](int buf, int slice, int into) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-            af[into][i] = *(const f16x8 *)(As(buf) + (wm * WM + i * 32 + lane % 32) * kLdsRow + slice * 16 +
-                                           (lane / 32) * 8);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-            bf[into][j] = *(const f16x8 *)(Bs(buf) + (wn * WN + j * 32 + lane % 32) * kLdsRow + slice * 16 +
-                                           (lane / 32) * 8);
-    };
-    auto mfmas = [&](int from) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[from][i], bf[from][j], acc[i][j], 0, 0, 0);
-    };
-    // One K step from LDS buffer `buf`. With LD, global loads of step `kload` go to register set LS during the first
-    // slice; with ST, register set SS is stored to the other LDS buffer during the last one. The group barriers lay
-    // the instruction stream out as MFMAs with the operand reads of the next slice, the global loads and the LDS
-    // stores threaded between them.
-    constexpr int NMF = TM * TN, NDR = TM + TN, NLD = AV + BV;
-    constexpr int LD_PER = (NLD + NMF - 1) / NMF;
-    auto step = [&](auto ld_tag, auto st_tag, auto ls_tag, auto ss_tag, int buf, uint32_t kload) {
-        constexpr bool LD = decltype(ld_tag)::value, ST = decltype(st_tag)::value;
-        frags(buf, 0, 0);
-        frags(buf, 1, 1);
-        if constexpr (LD)
-            load(ls_tag, kload);
-        mfmas(0);
-        frags(buf, 2, 0);
-        mfmas(1);
-        frags(buf, 3, 1);
-        mfmas(0);
-        mfmas(1);
-        if constexpr (ST)
-            stash(ss_tag, buf ^ 1);
-        // slice 0 operands first, then: slice 0 MFMAs with slice 1 reads and the global loads, slices 1 and 2 with
-        // the next slice's reads, slice 3 with the LDS stores
-        __builtin_amdgcn_sched_group_barrier(0x100, NDR, 0);
-#pragma unroll
-        for (int i = 0; i < NMF; ++i)
-        {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i < NDR)
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            if (LD && i * LD_PER < NLD)
-                __builtin_amdgcn_sched_group_barrier(0x020, LD_PER, 0);
-        }
-#pragma unroll
-        for (int sl = 1; sl < 3; ++sl)
-#pragma unroll
-            for (int i = 0; i < NMF; ++i)
-            {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                if (i < NDR)
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            }
-#pragma unroll
-        for (int i = 0; i < NMF; ++i)
-        {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (ST && i * LD_PER < NLD)
-                __builtin_amdgcn_sched_group_barrier(0x200, LD_PER, 0);
-        }
-    };
+    auto next_slot = [&](uint32_t o, uint32_t by) { return o + by >= NH * HALF ? o + by - NH * HALF : o + by; };
 
-    using T = std::true_type;
-    using F = std::false_type;
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, PF - 1>;
-    const uint32_t nsteps = (ke - kb) / kBK;
-    if constexpr (PF == 1)
+    for_seq(std::make_integer_sequence<int, NH - 1>{}, [&](auto j) {
+        constexpr int J = decltype(j)::value;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+            copy(std::integral_constant<int, J % 2>{}, i, J * HALF, kat(J));
+    });
+    // halves 0 and 1 have landed in every wave
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NH - 3) * ND) : "memory");
+#pragma unroll
+    for (int x = 0; x < NR; ++x)
+        read(I0{}, x / (TM + TN), x % (TM + TN), 0);
+    uint32_t slot = (NH - 1) * HALF;
+    for (uint32_t s = 0; s < nsteps; s += 2)
     {
-        load(S0{}, kb);
-        stash(S0{}, 0);
-        __syncthreads();
-        int cur = 0;
-        uint32_t k0 = kb;
-        for (; k0 + kBK < ke; k0 += kBK)
-        {
-            step(T{}, T{}, S0{}, S0{}, cur, k0 + kBK);
-            __syncthreads();
-            cur ^= 1;
-        }
-        step(F{}, F{}, S0{}, S0{}, cur, k0);
+        step(I0{}, I1{}, std::integral_constant<int, (NH - 1) % 2>{}, slot, kat(s + NH - 1));
+        slot = next_slot(slot, HALF);
+        // of the halves requested so far all but the last NH - 4 have landed, halves s + 2 and s + 3 among them, and
+        // every wave has read all of halves s and s + 1
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NH - 4) * ND) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        slot_a = next_slot(slot_a, 2 * HALF);
+        slot_b = next_slot(slot_b - WM * 128, 2 * HALF) + WM * 128;
+        step(I1{}, I0{}, std::integral_constant<int, NH % 2>{}, slot, kat(s + NH));
+        slot = next_slot(slot, HALF);
     }
-    else if constexpr (PF > 2)
-    {
-        // Step s computes from LDS buffer s % 2 while register sets hold steps s + 1 .. s + PF - 1 in flight: it
-        // loads step s + PF into set s % PF (free since step s went to LDS) and stores set (s + 1) % PF into buffer
-        // (s + 1) % 2. Loads past the last step re-read the last step (L2 hits), so every step is the same code and
-        // the wait before each store covers only the set being stored. Steps run in groups of PF (static set
-        // indices), the last nsteps % PF in a tail of straight-line steps.
-        static_assert(PF % 2 == 0, "PF > 2 must be even (buffer parity follows the set index)");
-        const uint32_t lastk = kb + (nsteps - 1) * kBK;
-        auto kat = [&](uint32_t st) { return st < nsteps ? kb + st * kBK : lastk; };
-        for_seq(std::make_integer_sequence<int, PF>{}, [&](auto j) { load(j, kat(decltype(j)::value)); });
-        stash(S0{}, 0);
-        __syncthreads();
-        uint32_t s = 0;
-        auto run_steps = [&](auto seq) {
-            for_seq(seq, [&](auto j) {
-                constexpr int J = decltype(j)::value;
-                step(T{}, T{}, j, std::integral_constant<int, (J + 1) % PF>{}, J % 2, kat(s + J + PF));
-                __syncthreads();
-            });
-        };
-        for (; s + PF <= nsteps; s += PF)
-            run_steps(std::make_integer_sequence<int, PF>{});
-        const uint32_t left = nsteps - s;
-        if constexpr (PF >= 4)
-        {
-            if (left == 3)
-                run_steps(std::make_integer_sequence<int, 3>{});
-            else if (left == 2)
-                run_steps(std::make_integer_sequence<int, 2>{});
-            else if (left == 1)
-                run_steps(std::make_integer_sequence<int, 1>{});
-        }
-        static_assert(PF <= 4, "tail covers at most 3 steps");
-    }
-    else
-    {
-        // step s computes from LDS buffer s % 2, loads step s + 2 into register set s % 2 and stores set
-        // (s + 1) % 2 (step s + 1, loaded during step s - 1) into buffer (s + 1) % 2; pairs keep the sets static
-        load(S0{}, kb);
-        load(S1{}, nsteps > 1 ? kb + kBK : kb); // unconditional: storing set 0 then waits for set 0 only
-        stash(S0{}, 0);
-        __syncthreads();
-        uint32_t s = 0;
-        for (; s + 3 < nsteps; s += 2)
-        {
-            step(T{}, T{}, S0{}, S1{}, 0, kb + (s + 2) * kBK);
-            __syncthreads();
-            step(T{}, T{}, S1{}, S0{}, 1, kb + (s + 3) * kBK);
-            __syncthreads();
-        }
-        const uint32_t left = nsteps - s; // 1, 2 or 3 steps, the first from buffer 0
-        if (left == 3)
-        {
-            step(T{}, T{}, S0{}, S1{}, 0, kb + (s + 2) * kBK);
-            __syncthreads();
-            step(F{}, T{}, S1{}, S0{}, 1, 0);
-            __syncthreads();
-            step(F{}, F{}, S0{}, S0{}, 0, 0);
-        }
-        else if (left == 2)
-        {
-            step(F{}, T{}, S0{}, S1{}, 0, 0);
-            __syncthreads();
-            step(F{}, F{}, S1{}, S1{}, 1, 0);
-        }
-        else
-            step(F{}, F{}, S0{}, S0{}, 0, 0);
-    }
+    // the copies past the end have landed before the ring is used again
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
     if constexpr (!SPLIT)
     {
-        // Epilogue through LDS (the K-step buffers are free now): each lane writes its fp16 outputs into a row-major
+        // Epilogue through LDS (the ring is free now): each lane writes its fp16 outputs into a row-major
         // tile, then the workgroup moves 16-byte row chunks to their destinations, so the stores (and the residual's
         // loads) are whole vectors instead of one 2-byte element per lane. SwiGLU tiles have BN / 2 output columns.
         constexpr int OC = is_dual(EPI) ? BN / 2 : BN;
         constexpr int TROW = OC + 8; // halves; rows 4 apart then start 16 banks apart
-        static_assert(BM * TROW <= 2 * (BM + BN) * kLdsRow, "epilogue tile fits the K-step buffers");
-        __syncthreads();
+        static_assert(BM * TROW * 2 <= NH * HALF, "epilogue tile fits the ring");
         uint16_t *T = lds;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; j += (is_dual(EPI) ? 2 : 1))
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
+                for (int e = 0; e < 16; e += is_dual(EPI) ? 2 : 1)
                 {
                     const uint32_t rt = wm * WM + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
                     const uint32_t ct = wn * WN + j * 32 + lane % 32;
                     if constexpr (is_dual(EPI))
-                        T[rt * TROW + swiglu_col(ct)] = dual_out<EPI>(acc[i][j][e], acc[i][j + 1][e]);
+                    {
+                        // Lanes 0-15 of each 32 hold up values and 16-31 the gate values of the same columns. Swapping
+                        // rows of 16 lanes between elements e and e + 1 leaves both values of element e in the first 16
+                        // and of e + 1 in the others, so every lane forms one output.
+                        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][j][e]),
+                                                                        __float_as_uint(acc[i][j][e + 1]), false, false);
+                        T[(rt + lane / 16 % 2) * TROW + swiglu_col(ct & ~16u)] =
+                            dual_out<EPI>(__uint_as_float(p[0]), __uint_as_float(p[1]));
+                    }
                     else if constexpr (EPI == GEMM_SILU_HI)
                         T[rt * TROW + ct] = f2h(n_base + n0 + ct >= split ? silu(acc[i][j][e]) : acc[i][j][e]);
                     else
@@ -509,6 +439,43 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
         // end of this launch's columns
         const uint32_t oce = is_dual(EPI) ? min((n_base + N) / 2, split) : n_base + N;
         const bool vec = ((uintptr_t)C % 16 == 0) && ldc % 8 == 0;
+        if (vec && oc0 + OC <= oce)
+        {
+            // Whole chunks: in batches whose loads (residuals, rotation angles) are requested together, since with one
+            // workgroup on the CU each would otherwise cost its full latency. Rows past M repeat the last one.
+            constexpr int IT = BM * CH / 256;
+            constexpr int U = IT % 8 == 0 ? 8 : IT % 6 == 0 ? 6 : IT % 5 == 0 ? 5 : IT % 4 == 0 ? 4 : IT % 3 == 0 ? 3 : 2;
+            static_assert(BM * CH % 256 == 0 && IT % U == 0, "whole batches");
+            for (int it = 0; it < IT; it += U)
+            {
+                u32x4 old[U];
+                Rope8 cs[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                {
+                    const uint32_t idx = tid + 256 * (it + u), m = min(m0 + idx / CH, M - 1), col = oc0 + (idx % CH) * 8;
+                    if constexpr (EPI == GEMM_QKV_ROPE)
+                        cs[u] = rope_load8(rope, m, col);
+                    if constexpr (EPI == GEMM_RESID)
+                        old[u] = *(const u32x4 *)(C + (size_t)m * ldc + col);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                {
+                    const uint32_t idx = tid + 256 * (it + u), m = m0 + idx / CH, col = oc0 + (idx % CH) * 8;
+                    u32x4 v = *(const u32x4 *)(T + (idx / CH) * TROW + (idx % CH) * 8);
+                    if constexpr (EPI == GEMM_RESID)
+                        v = resid8(old[u], v);
+                    if (m >= M)
+                        continue;
+                    if constexpr (EPI == GEMM_QKV_ROPE)
+                        rope_store8(rope, m, col, v, cs[u]);
+                    else
+                        *(u32x4 *)(C + (size_t)m * ldc + col) = v;
+                }
+            }
+            return;
+        }
         for (uint32_t idx = tid; idx < (uint32_t)(BM * CH); idx += 256)
         {
             const uint32_t rt = idx / CH, m = m0 + rt, col = oc0 + (idx % CH) * 8;
@@ -516,24 +483,13 @@ __global__ __launch_bounds__(256, (PF > 2 ? 1 : PF)) void gemm32_kernel(const ui
                 continue;
             const uint16_t *t = T + rt * TROW + (idx % CH) * 8;
             if constexpr (EPI == GEMM_QKV_ROPE)
-                rope_store8(rope, m, col, *(const u32x4 *)t); // N is a multiple of 64: whole chunks
+                rope_store8(rope, m, col, *(const u32x4 *)t, rope_load8(rope, m, col)); // N % 64 == 0: whole chunks
             else
             {
                 uint16_t *c = C + (size_t)m * ldc + col;
                 const uint32_t cnt = min(8u, oce - col);
                 if (vec && cnt == 8)
-                {
-                    u32x4 v = *(const u32x4 *)t;
-                    if constexpr (EPI == GEMM_RESID)
-                    {
-                        const u32x4 r = *(const u32x4 *)c;
-#pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            v[k] = pack2(f2h(h2f((uint16_t)r[k]) + half_lo(v[k])),
-                                         f2h(h2f((uint16_t)(r[k] >> 16)) + half_hi(v[k])));
-                    }
-                    *(u32x4 *)c = v;
-                }
+                    *(u32x4 *)c = EPI == GEMM_RESID ? resid8(*(const u32x4 *)c, *(const u32x4 *)t) : *(const u32x4 *)t;
                 else
                     for (uint32_t k = 0; k < cnt; ++k)
                         c[k] = EPI == GEMM_RESID ? f2h(h2f(c[k]) + h2f(t[k])) : t[k];
@@ -600,23 +556,23 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 h[k] = pack2(f2h(v[2 * k]), f2h(v[2 * k + 1]));
-            rope_store8(rope, m, n_base + n, h);
+            rope_store8(rope, m, n_base + n, h, rope_load8(rope, m, n_base + n));
         }
         return;
     }
     if constexpr (is_dual(EPI))
     {
-        // 8 output columns f..f + 7 (inside one 32-column block): up columns c..c + 7, gate columns c + 32..c + 39
+        // 8 output columns f..f + 7 (inside one 16-column block): up columns c..c + 7, gate columns c + 16..c + 23
         const uint32_t per_row = N / 16;
         const uint64_t chunks = (uint64_t)M * per_row;
         for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < chunks; i += (uint64_t)gridDim.x * 256)
         {
-            const uint32_t m = (uint32_t)(i / per_row), f = 8 * (uint32_t)(i % per_row), c = 64 * (f / 32) + f % 32;
+            const uint32_t m = (uint32_t)(i / per_row), f = 8 * (uint32_t)(i % per_row), c = 32 * (f / 16) + f % 16;
             if (n_base / 2 + f >= split) // columns past F (GEMM_FFN with F % 32 != 0)
                 continue;
             float up[8], gate[8];
             sum8((size_t)m * N + c, up);
-            sum8((size_t)m * N + c + 32, gate);
+            sum8((size_t)m * N + c + 16, gate);
             u32x4 o;
 #pragma unroll
             for (int k = 0; k < 4; ++k)
@@ -848,19 +804,19 @@ static hipError_t launch_tile(hipStream_t st, const uint16_t *A, const uint16_t 
     return hipGetLastError();
 }
 
-template <int BM, int BN, int EPI, bool SPLIT, int PF = 1>
+template <int BM, int BN, int EPI, bool SPLIT>
 static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                 uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
                                 uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
 {
     static uint64_t attr_devs = 0; // devices on which the LDS limit is raised for this kernel
-    const size_t lds = gemm_lds<BM, BN>();
-    hipError_t e = lds_attr_once((const void *)gemm32_kernel<BM, BN, EPI, SPLIT, PF>, lds, attr_devs);
+    const size_t lds = (size_t)gemm_ring<BM, BN>() * (BM + BN) * 64;
+    hipError_t e = lds_attr_once((const void *)gemm32_kernel<BM, BN, EPI, SPLIT>, lds, attr_devs);
     if (e != hipSuccess)
         return e;
     const uint32_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, total = tm * tn;
     const uint32_t grid = (total + 7) / 8 * 8;
-    gemm32_kernel<BM, BN, EPI, SPLIT, PF><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
+    gemm32_kernel<BM, BN, EPI, SPLIT><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
         A, B.p, B.p2, C, work, M, N, K, ldc, split, kchunk, tm, total, n_base, rope ? *rope : GemmRope{});
     return hipGetLastError();
 }
@@ -876,22 +832,6 @@ static hipError_t launch_reduce(hipStream_t st, const float *work, uint16_t *C, 
 }
 
 template <int BM, int BN, int EPI>
-static hipError_t launch_shape32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
-                                 uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
-                                 uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
-{
-    if (splits <= 1)
-        return launch_tile32<BM, BN, EPI, false>(st, A, B, C, work, M, N, K, ldc, split, 1, K, n_base, rope);
-    // split tiles (short prompts): two K steps of loads in flight where the registers allow it
-    constexpr int PF = BM * BN <= 128 * 128 ? 2 : 1;
-    hipError_t e = launch_tile32<BM, BN, EPI, true, PF>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk,
-                                                        n_base, rope);
-    if (e != hipSuccess)
-        return e;
-    return launch_reduce<EPI>(st, work, C, M, N, ldc, split, splits, n_base, rope);
-}
-
-template <int BM, int BN, int EPI>
 static hipError_t launch_shape(hipStream_t st, const uint16_t *A, const uint16_t *B, uint16_t *C, float *work,
                                uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
                                uint32_t kchunk)
@@ -904,6 +844,81 @@ static hipError_t launch_shape(hipStream_t st, const uint16_t *A, const uint16_t
     const uint32_t grid = reduce_grid<EPI>(M, N, ldc, 0, C);
     gemm_splitk_reduce_kernel<EPI><<<grid, 256, 0, st>>>(work, C, M, N, ldc, split, splits, 0, GemmRope{});
     return hipGetLastError();
+}
+
+// ---- tile and split of a product ----
+struct TileShape
+{
+    uint16_t bm, bn;
+    float step_us; // 64 of K on one of many busy CUs, measured (products of 64 to 216 such steps in one round)
+};
+constexpr TileShape kTiles[] = {{256, 256, 1.29f}, {256, 192, 1.18f}, {256, 128, 0.88f}, {128, 320, 1.18f},
+                                {320, 128, 1.05f}, {192, 128, 0.66f}, {128, 128, 0.50f}, {64, 128, 0.36f}};
+constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+
+template <int EPI, bool SPLIT>
+static hipError_t launch_choice(hipStream_t st, int tile, const uint16_t *A, GemmB B, uint16_t *C, float *work, uint32_t M,
+                                uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits, uint32_t kchunk,
+                                const GemmRope *rope)
+{
+    hipError_t e = hipErrorInvalidValue;
+    for_seq(std::make_integer_sequence<int, kTileCount>{}, [&](auto i) {
+        constexpr TileShape T = kTiles[decltype(i)::value];
+        if (tile == decltype(i)::value)
+            e = launch_tile32<T.bm, T.bn, EPI, SPLIT>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, 0, rope);
+    });
+    return e;
+}
+
+struct TileChoice
+{
+    int tile;
+    uint32_t splits;
+};
+
+// Time of a product on one tile shape with K in `splits` ranges, us: the tile's measured step, or what the busy CUs
+// together sustain (1.3 PFLOP/s); each round of workgroups adds its start and its epilogue, split K the partials written
+// and read and the reduce's launch, whole K the RMSNorm pass that the reduce would have included; and the weights come
+// from HBM at 4.6 TB/s, or 24 bytes/ns of each workgroup. Over 73 products of 16 to 2048 rows at the 7B and 13B widths the choice made from it is the
+// fastest measured one or within 11% of it in all but 4.
+static float tile_time(uint32_t M, uint32_t N, uint32_t K, TileShape t, uint32_t splits, uint32_t cus, bool norm)
+{
+    const uint64_t wgs = (uint64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * splits;
+    const uint32_t steps = (K / kBK + splits - 1) / splits;
+    const float flop = 2.f * t.bm * t.bn * kBK, area = t.bm * t.bn / 65536.f;
+    auto round = [&](float n) { return steps * std::max(t.step_us, n * flop / 1.3e9f) + 5.f + 5.f * area; };
+    const uint64_t full = wgs / cus, rest = wgs % cus;
+    float us = full * round((float)cus) + (rest ? round((float)rest) : 0.f);
+    // several rows of tiles share the weights through L2 at some cost; the last term: of tiles that all wait for the
+    // weights, the one that is done soonest
+    const float weights = (float)N * K * 2 * (M > t.bm ? 1.2f : 1.f);
+    us = std::max(us, 3.f + weights / std::min(4.6e6f, 2.4e4f * wgs)) + 0.05f * us;
+    const float mn = (float)M * N;
+    if (splits > 1)
+        us += 4.f + splits * mn * 4 / 3.5e6f;
+    else if (norm)
+        us += 4.f + mn * 4 / 3.5e6f;
+    return us;
+}
+
+static TileChoice pick_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, size_t work_elems, bool norm)
+{
+    TileChoice best{0, 1};
+    float best_us = FLT_MAX;
+    for (int i = 0; i < kTileCount; ++i)
+        for (uint32_t s = 1; s <= 16; ++s)
+        {
+            // a range keeps at least 256 of K
+            if (s > 1 && (K / s < 4 * kBK || (size_t)s * M * N > work_elems))
+                break;
+            const float us = tile_time(M, N, K, kTiles[i], s, cus, norm);
+            if (us < best_us)
+            {
+                best_us = us;
+                best = {i, s};
+            }
+        }
+    return best;
 }
 
 template <int EPI>
@@ -925,103 +940,23 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
             return hipErrorInvalidValue;
     if (K % kBK == 0)
     {
-        // 32x32x16 kernel: 256 x 256 tiles when they alone give most CUs a tile; else 128 x 128 tiles (two fit a
-        // CU) with K split until about two workgroups per CU run, or 1.4 for prompts of at most 128 tokens (their
-        // partial tiles cost more than further splits gain), each split keeping at least 256 of K
-        const uint64_t t256 = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
-        // also when 128 x 128 tiles would take more rounds: a pair of them on a CU takes about 2/3 of a 256 x 256
-        // tile's time (13B Wo and down at 2048 tokens: 160 tiles, 141 and 395 us against 189 and 514 us)
-        const uint64_t r256 = (t256 + cus - 1) / cus, r128 = (2 * t256 + cus - 1) / cus;
-        if (t256 >= (cus * 3) / 4 || r128 * 2 > r256 * 3)
-        {
-            // Residual products whose 256 x 256 tiles make one partial round: 128 x 320 tiles when they give at
-            // least 1.5 times as many CUs a tile in one round (13B Wo and down at 2048 tokens: 256 tiles for 256
-            // CUs instead of 160; Wo + Wd 528 -> 485 us per layer, outputs bit-identical, since every output adds its
-            // K terms in the same order in either tile). The same tiles were slower for the plain vocabulary product,
-            // and 128 x 384 tiles level for the 7B QKV product at 1024 tokens.
-            if constexpr (EPI == GEMM_RESID)
-            {
-                const uint64_t t320 = (uint64_t)((M + 127) / 128) * ((N + 319) / 320);
-                if (t256 < cus && t320 <= cus && t320 * 2 >= t256 * 3)
-                    return launch_tile32<128, 320, EPI, false, 1>(st, A, B, C, work, M, N, K, ldc, split, 1, K);
-            }
-            // A last round of 256 x 256 tiles at most half full would leave most CUs idle for a whole tile's time:
-            // its tile columns run as a product of their own with K split over those CUs (partials added in order
-            // by the reduce), the full rounds as before.
-            const uint32_t tm = (M + 255) / 256, tn = (N + 255) / 256;
-            const uint64_t full = t256 / cus, rem = t256 % cus;
-            if (full >= 1 && rem > 0 && rem * 2 <= cus)
-            {
-                const uint32_t tail_cols = (uint32_t)((rem + tm - 1) / tm), n_split = (tn - tail_cols) * 256;
-                const uint32_t tail_n = N - n_split;
-                uint32_t splits = cus / (tm * tail_cols);
-                while (splits > 1 && (K / splits < 4 * kBK || (size_t)splits * M * tail_n > work_elems))
-                    --splits;
-                if (splits >= 2)
-                {
-                    const uint32_t kchunk = ((K + splits - 1) / splits + kBK - 1) / kBK * kBK;
-                    hipError_t e =
-                        launch_shape32<256, 256, EPI>(st, A, B, C, work, M, n_split, K, ldc, split, 1, K, 0, rope);
-                    if (e != hipSuccess)
-                        return e;
-                    return launch_shape32<256, 256, EPI>(st, A, B, C, work, M, tail_n, K, ldc, split,
-                                                         (K + kchunk - 1) / kchunk, kchunk, n_split, rope);
-                }
-            }
-            return launch_shape32<256, 256, EPI>(st, A, B, C, work, M, N, K, ldc, split, 1, K, 0, rope);
-        }
-        // Residual products of long rows (K >= 5120: 13B Wo, 7B and 13B down) above 128 tokens whose 256 x 256 tiles
-        // leave most CUs idle: K split s ways so that one round of 256 x 256 tiles fills at least three quarters of
-        // the CUs, each split keeping at least 1280 of K. Against the 128 x 128 path: 7B down at 1024 tokens 110 vs
-        // 135 us (4 splits), 13B down 145 vs 250 us (3), 13B Wo 84 vs 108 us (3), 7B down at 640 tokens 92 vs 127 us
-        // (5), 7 to 30% at 384-2048 tokens; 7B Wo (K 4096) is level or slower at every length and stays on 128 x 128.
+        const TileChoice c = pick_tile(M, N, K, cus, work_elems, EPI == GEMM_RESID && norm);
+        const uint32_t kchunk = ((K + c.splits - 1) / c.splits + kBK - 1) / kBK * kBK, splits = (K + kchunk - 1) / kchunk;
+        if (splits <= 1)
+            return launch_choice<EPI, false>(st, c.tile, A, B, C, nullptr, M, N, K, ldc, split, 1, K, rope);
+        // the partial tiles are the same for every epilogue: one kernel for products of one matrix, one for dual ones
+        constexpr int PART = is_dual(EPI) ? GEMM_SWIGLU : GEMM_PLAIN;
+        hipError_t e = launch_choice<PART, true>(st, c.tile, A, B, C, work, M, N, K, ldc, split, splits, kchunk, nullptr);
+        if (e != hipSuccess)
+            return e;
         if constexpr (EPI == GEMM_RESID)
-        {
-            const uint32_t s = t256 > 0 ? (uint32_t)(cus / t256) : 0;
-            if (M > 128 && K >= 5120 && s >= 2 && t256 * s * 4 >= (uint64_t)cus * 3 && K / s >= 1280 &&
-                (size_t)s * M * N <= work_elems)
-            {
-                const uint32_t kchunk = ((K + s - 1) / s + kBK - 1) / kBK * kBK, ns = (K + kchunk - 1) / kchunk;
-                hipError_t e =
-                    launch_tile32<256, 256, EPI, true, 1>(st, A, B, C, work, M, N, K, ldc, split, ns, kchunk);
-                if (e != hipSuccess)
-                    return e;
-                if (norm)
-                {
-                    *normed = true;
-                    return launch_resid_norm(st, work, C, M, N, ns, *norm);
-                }
-                return launch_reduce<EPI>(st, work, C, M, N, ldc, split, ns, 0, nullptr);
-            }
-        }
-        const uint64_t tiles = (uint64_t)((M + 127) / 128) * ((N + 127) / 128);
-        // prompts of at most 128 tokens whose tiles cover two thirds of the CUs or more ([Wu;Wg], logits): the
-        // whole K per tile with four K steps of loads in flight (one workgroup per CU) beats split K and its reduce
-        if (M <= 128 && tiles * 3 >= (uint64_t)cus * 2)
-            return launch_tile32<128, 128, EPI, false, 4>(st, A, B, C, work, M, N, K, ldc, split, 1, K, 0, rope);
-        // workgroups per CU, times 10. Plain products above 128 tokens (the MATMUL op's) split K only until one
-        // workgroup per CU runs: a second workgroup per CU leaves the tile kernel no faster and doubles the partials
-        // the reduce reads (M 512, N = K = 4096: 128 tiles x 2 K ranges 29.7 + 5.4 us, x 4 ranges 30.2 + 8.2 us)
-        const uint64_t per_cu10 = M <= 128 ? 14 : EPI == GEMM_PLAIN ? 10 : 20;
-        uint32_t splits = 1;
-        while (tiles * splits * 2 * 10 <= per_cu10 * cus && K / (splits * 2) >= 256 &&
-               (size_t)splits * 2 * M * N <= work_elems)
-            splits *= 2;
-        const uint32_t kchunk = ((K + splits - 1) / splits + kBK - 1) / kBK * kBK;
-        splits = (K + kchunk - 1) / kchunk;
-        if constexpr (EPI == GEMM_RESID)
-            if (norm && splits > 1)
+            if (norm)
             {
                 // the reduce adds the residual and normalises the updated rows in one pass
-                hipError_t e = launch_tile32<128, 128, EPI, true, 2>(st, A, B, C, work, M, N, K, ldc, split, splits,
-                                                                     kchunk);
-                if (e != hipSuccess)
-                    return e;
-                // 512 threads a row (one 16-byte vector each at width 4096) keep a row's partial loads in flight
                 *normed = true;
                 return launch_resid_norm(st, work, C, M, N, splits, *norm);
             }
-        return launch_shape32<128, 128, EPI>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, 0, rope);
+        return launch_reduce<EPI>(st, work, C, M, N, ldc, split, splits, 0, rope);
     }
     if constexpr (is_dual(EPI) || EPI == GEMM_QKV_ROPE)
         return hipErrorInvalidValue; // checked above: not reached
