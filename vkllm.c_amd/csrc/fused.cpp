@@ -28,6 +28,7 @@ struct FusedPlan
     uint32_t offset;
     uint32_t S;
     bool ran = false; // fused_plan_run enqueued (and completed) the step
+    bool last = false; // the caller says that no step at the next position follows
 };
 
 // Short-cache decode steps are captured per bucket of kSmallBucket cache positions: a bucket's launches bound their
@@ -221,6 +222,11 @@ void *fused_plan_new(vkllm_models_llama2 *model, vkllm_tensor *input_toks, uint3
     p->offset = offset;
     p->S = input_toks->shapes[3];
     return p;
+}
+
+void fused_plan_last_step(void *plan)
+{
+    ((FusedPlan *)plan)->last = true;
 }
 
 bool fused_plan_ran(const void *plan)
@@ -1101,7 +1107,7 @@ vkllm_err_t fused_plan_run(vkllm_context *ctx, vkllm_graph *graph)
             HIP_TRY(hipEventRecord(fs->slot_done[slot], st));
         }
         fs->ahead_live = false;
-        if (fs->ahead_enabled && !direct && p->offset + 1 < mp->ctx)
+        if (fs->ahead_enabled && !p->last && !direct && p->offset + 1 < mp->ctx)
         {
             // the step at p + 1 behind this one, its token this step's device-side arg max
             const int nx = 1 - slot;
