@@ -294,6 +294,21 @@ hipError_t launch_gemm(hipStream_t st, int epi, const uint16_t *A, const uint16_
                        uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, int cu_count, float *work,
                        size_t work_elems, const GemmRope *rope = nullptr, const GemmNorm *norm = nullptr,
                        const uint16_t *B2 = nullptr);
+// The same for small models, one launch with the RMSNorm of A's rows in front (norm_w): GEMM_PLAIN, GEMM_SWIGLU (B up
+// rows, B2 gate rows, N = F) and GEMM_QKV_ROPE with it, GEMM_RESID and GEMM_FFN without. C is [M, N] packed, rows
+// 16-byte aligned in A and B, N even, K % 32 == 0 and at most kGemmSmallMaxK; the head size even.
+constexpr uint32_t kGemmSmallMaxK = 1024;
+struct GemmSmallArgs
+{
+    const uint16_t *A, *B, *B2;
+    uint16_t *C;
+    const float *norm_w;
+    float eps;
+    uint32_t M, N, K;
+    GemmRope rope;
+};
+bool gemm_small_ok(uint32_t M, uint32_t N, uint32_t K);
+hipError_t launch_gemm_small(hipStream_t st, int epi, const GemmSmallArgs &g);
 // Prompt-step products of at most 128 tokens with the weights read from a fragment-tiled copy (launch_tile_weights)
 // and X fragment-ordered (xt_vec): C[M, N] = X[M, K] . W[N, K]^T, M <= 128, K % 16 == 0.
 enum StreamEpi : int

@@ -647,8 +647,17 @@ extern "C" vkllm_err_t vkllm_op_ffn_up_and_gate_init(struct vkllm_context *conte
 // the 22 vectors a lane holds of a row), more on the tile GEMM (K in whole 64-wide steps). Both sum in fp32 and round
 // the product once, as the generic kernel does. 7B widths: 512 rows 2756 us on the generic kernel (vector FMAs from
 // 64 x 64 LDS tiles), 119 us on the tile GEMM (92 GFLOP, 776 TFLOP/s; 172 of 256 CUs hold a tile); one row 27.7 us on
-// the GEMV, 6.5 TB/s of weights.
-static bool ffn_fast_path(const vk::TView &x, const vk::TView &wu, const vk::TView &wg, const vk::TView &out)
+// the GEMV, 6.5 TB/s of weights. Small products of other K (whole 32-wide steps) take the one-launch kernel of small
+// models: 16 rows of the tiny decoder's widths (288 to 768) 69 -> 3.3 us, 200 rows 81 -> 4.4.
+enum class FfnPath
+{
+    GENERIC,
+    ROW,
+    TILES,
+    SMALL
+};
+
+static FfnPath ffn_path(const vk::TView &x, const vk::TView &wu, const vk::TView &wg, const vk::TView &out)
 {
     auto packed = [](const vk::TView &v) {
         return v.dt == vkllm_dtype_float16 && v.s[3] == 1 && v.s[2] == v.n[3] && v.s[1] == v.n[2] * v.s[2] &&
@@ -657,10 +666,12 @@ static bool ffn_fast_path(const vk::TView &x, const vk::TView &wu, const vk::TVi
     const uint64_t rows = (uint64_t)x.n[0] * x.n[1] * x.n[2];
     const uint32_t K = x.n[3], F = out.n[3];
     if (!packed(x) || !packed(wu) || !packed(wg) || !packed(out) || rows == 0 || rows > 0x7fffffffu || F == 0)
-        return false;
-    if (rows == 1)
-        return K % 8 == 0 && K <= 8 * 64 * 22;
-    return K > 0 && K % 64 == 0 && F % 8 == 0 && 2ull * F * K < (1ull << 32) - 64ull * K;
+        return FfnPath::GENERIC;
+    if (rows == 1 && K % 8 == 0 && K > 0 && K <= 8 * 64 * 22)
+        return FfnPath::ROW;
+    if (K > 0 && K % 64 == 0 && F % 8 == 0 && 2ull * F * K < (1ull << 32) - 64ull * K)
+        return FfnPath::TILES;
+    return rows <= 256 && vk::gemm_small_ok((uint32_t)rows, F, K) ? FfnPath::SMALL : FfnPath::GENERIC;
 }
 
 static hipError_t launch_op_ffn_row(vkllm_context *ctx, const vk::TView &x, const vk::TView &wu, const vk::TView &wg,
@@ -692,21 +703,24 @@ extern "C" vkllm_err_t vkllm_op_ffn_up_and_gate_run(struct vkllm_context *contex
     NEED_DEV(out);
     const uint32_t K = x.n[3], F = out.n[3];
     const uint64_t rows = (uint64_t)x.n[0] * x.n[1] * x.n[2];
-    if (ffn_fast_path(x, wu, wg, out))
+    const FfnPath path = ffn_path(x, wu, wg, out);
+    if (path == FfnPath::ROW)
+        LAUNCH(context, KID_FFN, launch_op_ffn_row(context, x, wu, wg, out));
+    else if (path == FfnPath::SMALL)
+        LAUNCH(context, KID_FFN,
+               vk::launch_gemm_small(context->device->stream, vk::GEMM_FFN,
+                                     vk::GemmSmallArgs{(const uint16_t *)x.p, (const uint16_t *)wu.p,
+                                                       (const uint16_t *)wg.p, (uint16_t *)out.p, nullptr, 0.f,
+                                                       (uint32_t)rows, F, K, vk::GemmRope{}}));
+    else if (path == FfnPath::TILES)
     {
-        if (rows == 1)
-            LAUNCH(context, KID_FFN, launch_op_ffn_row(context, x, wu, wg, out));
-        else
-        {
-            float *work = nullptr;
-            size_t work_elems = 0;
-            _CHECK(op_gemm_workspace(context, &work, &work_elems));
-            LAUNCH(context, KID_FFN,
-                   vk::launch_gemm(context->device->stream, vk::GEMM_FFN, (const uint16_t *)x.p, (const uint16_t *)wu.p,
-                                   (uint16_t *)out.p, (uint32_t)rows, (2 * F + 63) / 64 * 64, K, F, F,
-                                   context->device->cu_count, work, work_elems, nullptr, nullptr,
-                                   (const uint16_t *)wg.p));
-        }
+        float *work = nullptr;
+        size_t work_elems = 0;
+        _CHECK(op_gemm_workspace(context, &work, &work_elems));
+        LAUNCH(context, KID_FFN,
+               vk::launch_gemm(context->device->stream, vk::GEMM_FFN, (const uint16_t *)x.p, (const uint16_t *)wu.p,
+                               (uint16_t *)out.p, (uint32_t)rows, (2 * F + 63) / 64 * 64, K, F, F,
+                               context->device->cu_count, work, work_elems, nullptr, nullptr, (const uint16_t *)wg.p));
     }
     else
         LAUNCH(context, KID_FFN, vk::launch_ffn_up_and_gate(context->device->stream, x, wu, wg, out));
