@@ -24,11 +24,13 @@ namespace vk
 
 // ---------------------------------------------------------------------------------------------------------------
 // EMBEDDING (src/shaders/vkllm_embedding.comp:41-70) for contiguous rows
-__global__ void embed_rows_kernel(const uint32_t *toks, const uint16_t *embd, uint16_t *h, uint32_t V, uint32_t D,
-                                  uint32_t unk)
+__global__ void embed_rows_kernel(const uint32_t *toks, Step now, Step *step, const uint16_t *embd, uint16_t *h,
+                                  uint32_t V, uint32_t D, uint32_t unk)
 {
     const uint32_t s = blockIdx.x;
     uint32_t tok = toks[s];
+    if (s == 0 && threadIdx.x == 0)
+        *step = now;
     if (tok >= V)
         tok = unk;
     u32x4 *dst = (u32x4 *)(h + (size_t)s * D);
@@ -44,10 +46,10 @@ __global__ void embed_rows_kernel(const uint32_t *toks, const uint16_t *embd, ui
         dst[i] = src[i];
 }
 
-hipError_t launch_embed_rows(hipStream_t st, const uint32_t *toks, uint32_t S, const uint16_t *embd, uint16_t *h,
-                             uint32_t V, uint32_t D, uint32_t unk)
+hipError_t launch_embed_rows(hipStream_t st, const uint32_t *toks, const Step &now, Step *step, const uint16_t *embd,
+                             uint16_t *h, uint32_t V, uint32_t D, uint32_t unk)
 {
-    embed_rows_kernel<<<S, 128, 0, st>>>(toks, embd, h, V, D, unk);
+    embed_rows_kernel<<<now.S, 128, 0, st>>>(toks, now, step, embd, h, V, D, unk);
     return hipGetLastError();
 }
 
@@ -1191,7 +1193,7 @@ hipError_t launch_swiglu(hipStream_t st, const uint16_t *ug, uint16_t *act, uint
 // ARG_MAX for contiguous fp16 rows, one pass: 16-byte loads, then wave shuffles and one LDS step under the
 // reference's arg-max order (am_before), which is a total order, so the reduction tree does not matter.
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t *logits, uint32_t *ids, uint32_t V,
-                                                           DecodeIo *io)
+                                                           DecodeIo *io, uint32_t *host_ids)
 {
     __shared__ float wv[16];
     __shared__ uint32_t wi[16];
@@ -1281,17 +1283,19 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t *logit
                 bi = wi[w];
             }
         ids[blockIdx.x] = bi;
+        if (host_ids)
+            host_ids[blockIdx.x] = bi;
         if (io && blockIdx.x == 0)
             io->id = bi;
     }
 }
 
 hipError_t launch_argmax_rows(hipStream_t st, const uint16_t *logits, uint32_t *ids, uint32_t S, uint32_t V,
-                              DecodeIo *io)
+                              DecodeIo *io, uint32_t *host_ids)
 {
     if (S == 0 || V == 0)
         return hipErrorInvalidValue;
-    argmax_rows_kernel<<<S, 1024, 0, st>>>(logits, ids, V, io);
+    argmax_rows_kernel<<<S, 1024, 0, st>>>(logits, ids, V, io, host_ids);
     return hipGetLastError();
 }
 

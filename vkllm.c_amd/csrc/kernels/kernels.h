@@ -66,9 +66,9 @@ struct DecodeIo
 // *prev_id when io->token_dev is set
 hipError_t launch_embed_decode(hipStream_t st, const DecodeIo *io, Step *step, const uint16_t *embd, uint16_t *h,
                                uint32_t V, uint32_t D, uint32_t unk, const uint32_t *prev_id);
-// h[s] = embd[toks[s]] (ids >= V read row unk), s < S; D % 8 == 0
-hipError_t launch_embed_rows(hipStream_t st, const uint32_t *toks, uint32_t S, const uint16_t *embd, uint16_t *h,
-                             uint32_t V, uint32_t D, uint32_t unk);
+// *step = now, and h[s] = embd[toks[s]] (ids >= V read row unk), s < now.S; D % 8 == 0; toks in pinned or device memory
+hipError_t launch_embed_rows(hipStream_t st, const uint32_t *toks, const Step &now, Step *step, const uint16_t *embd,
+                             uint16_t *h, uint32_t V, uint32_t D, uint32_t unk);
 // y[s] = rmsnorm(x[s]) * w, s < S; with xt, y is fragment-ordered (xt_vec; S <= 128, D % 16 == 0)
 hipError_t launch_rmsnorm_rows(hipStream_t st, const uint16_t *x, const float *w, uint16_t *y, uint32_t S,
                                uint32_t D, float eps, bool xt = false);
@@ -248,9 +248,9 @@ hipError_t launch_rope_kv(hipStream_t st, const uint16_t *qkv, uint16_t *q, uint
 // act[s][n] = fp16(ug[s][n] * ug[s][F + n])
 hipError_t launch_swiglu(hipStream_t st, const uint16_t *ug, uint16_t *act, uint32_t S, uint32_t F);
 // ids[s] = arg_max(logits[s]) with the reference's tie rule, contiguous rows of V; with `io`, row 0's id also goes
-// to io->id
+// to io->id, and with `host_ids` (pinned) every id there as well
 hipError_t launch_argmax_rows(hipStream_t st, const uint16_t *logits, uint32_t *ids, uint32_t S, uint32_t V,
-                              DecodeIo *io = nullptr);
+                              DecodeIo *io = nullptr, uint32_t *host_ids = nullptr);
 
 enum GemmEpi : int
 {
