@@ -323,6 +323,16 @@ void fused_model_release(vkllm_context *ctx, vkllm_models_llama2 *model)
 // most 128 tokens (decode-only use never pays for them). Shapes the streamed products and their producers cannot
 // take, too little free memory, or a failed allocation leave stream_ok false: those steps then run on the row-major
 // slab.
+// Whether the vocabulary product of a short prompt streams its tiled weights. A workgroup streams 128 rows whatever
+// their number, in 27 us at 37 tokens and 40 us at 128 (K 4096), so few rows leave the chip idle for that long; the tile
+// GEMM splits K over it instead. us at 37 tokens, streamed / tiled: V 1000 28 / 14, 8192 30 / 20, 12288 31 / 29, 16000
+// 35 / 38 (at 128 tokens 40 / 15, 41 / 26, 43 / 34, 46 / 40). Below a width of 2048 the walk along K is short. The
+// streamed product stores 4 logits of a row as one 8-byte vector, so its rows of V must stay 8-byte aligned.
+static bool streams_logits(const ModelPriv *mp)
+{
+    return mp->V % 4 == 0 && (mp->V > 12288 || mp->D < 2048);
+}
+
 static vkllm_err_t build_stream_tiles(vkllm_context *ctx, ModelPriv *mp)
 {
     FusedState *fs = mp->fs;
@@ -336,7 +346,7 @@ static vkllm_err_t build_stream_tiles(vkllm_context *ctx, ModelPriv *mp)
         return VKLLM_ERR_OK;
     const size_t per_layer = vk::stream_tiled_elems(3 * D, D, 0) + vk::stream_tiled_elems(D, D, 0) +
                              vk::stream_tiled_elems(2 * F, D, F);
-    const size_t total = per_layer * mp->L + vk::stream_tiled_elems(V, D, 0);
+    const size_t total = per_layer * mp->L + (streams_logits(mp) ? vk::stream_tiled_elems(V, D, 0) : 0);
     size_t free_b = 0, total_b = 0;
     HIP_TRY(hipMemGetInfo(&free_b, &total_b));
     if (total * 2 + (size_t)2 * 128 * D * 2 > free_b / 2)
@@ -374,8 +384,11 @@ static vkllm_err_t build_stream_tiles(vkllm_context *ctx, ModelPriv *mp)
         HIP_TRY(vk::launch_tile_weights(st, ly.wug, t.wug, 2 * F, D, F));
         p += vk::stream_tiled_elems(2 * F, D, F);
     }
-    fs->out_t = p;
-    HIP_TRY(vk::launch_tile_weights(st, mp->out_w, fs->out_t, V, D, 0));
+    if (streams_logits(mp))
+    {
+        fs->out_t = p;
+        HIP_TRY(vk::launch_tile_weights(st, mp->out_w, fs->out_t, V, D, 0));
+    }
     HIP_TRY(hipStreamSynchronize(st));
     fs->stream_ok = true;
     return VKLLM_ERR_OK;
@@ -936,9 +949,8 @@ static vkllm_err_t enqueue_prefill(vkllm_context *ctx, ModelPriv *mp, uint32_t S
     // reading fragment-ordered activations (the normalised rows in xn_t, the attention output in attn_t)
     const bool streamed = fs->stream_ok && S <= 128 && rope_epi && fs->norm_epi;
     uint16_t *xn = streamed ? fs->xn_t : fs->xn;
-    // the streamed vocabulary product stores 4 logits of a row as one 8-byte vector, so its rows of V must stay
-    // 8-byte aligned; otherwise the tile GEMM takes the logits, and the last norm writes its row-major input
-    const bool stream_logits = streamed && V % 4 == 0;
+    // where the tile GEMM takes the logits, the last norm writes its row-major input
+    const bool stream_logits = streamed && streams_logits(mp);
     uint16_t *attn = streamed ? fs->attn_t : fs->attn;
     charge(ctx, fs, NS_ATTN_NORM, 0);
     KTRY(ctx, KID_F_RMSNORM, vk::launch_rmsnorm_rows(st, fs->h, mp->layers[0].attn_norm, xn, S, D, mp->eps, streamed));
