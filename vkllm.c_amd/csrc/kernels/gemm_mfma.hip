@@ -879,7 +879,7 @@ struct TileChoice
 // Time of a product on one tile shape with K in `splits` ranges, us: the tile's measured step, or what the busy CUs
 // together sustain (1.3 PFLOP/s); each round of workgroups adds its start and its epilogue, split K the partials written
 // and read and the reduce's launch, whole K the RMSNorm pass that the reduce would have included; and the weights come
-// from HBM at 4.6 TB/s, or 24 bytes/ns of each workgroup. Over 73 products of 16 to 2048 rows at the 7B and 13B widths the choice made from it is the
+// from HBM at 4.6 TB/s, or 24 bytes/ns of each workgroup (18 of a part of its rows). Over 73 products of 16 to 2048 rows at the 7B and 13B widths the choice made from it is the
 // fastest measured one or within 11% of it in all but 4.
 static float tile_time(uint32_t M, uint32_t N, uint32_t K, TileShape t, uint32_t splits, uint32_t cus, bool norm)
 {
@@ -892,7 +892,7 @@ static float tile_time(uint32_t M, uint32_t N, uint32_t K, TileShape t, uint32_t
     // several rows of tiles share the weights through L2 at some cost; the last term: of tiles that all wait for the
     // weights, the one that is done soonest
     const float weights = (float)N * K * 2 * (M > t.bm ? 1.2f : 1.f);
-    us = std::max(us, 3.f + weights / std::min(4.6e6f, 2.4e4f * wgs)) + 0.05f * us;
+    us = std::max(us, 3.f + weights / std::min(4.6e6f, (splits > 1 ? 1.8e4f : 2.4e4f) * wgs)) + 0.05f * us;
     const float mn = (float)M * N;
     if (splits > 1)
         us += 4.f + splits * mn * 4 / 3.5e6f;
