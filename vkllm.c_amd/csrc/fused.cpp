@@ -984,7 +984,7 @@ static vkllm_err_t enqueue_prefill(vkllm_context *ctx, ModelPriv *mp, uint32_t S
         }
         charge(ctx, fs, NS_SCORES, l);
         KTRY(ctx, KID_F_ATTN_PREFILL,
-             vk::launch_attn_prefill(st, fs->q, ly.kc, ly.vc, attn, offset, S, mp->H, hd, mp->ctx, scale, streamed));
+             vk::launch_attn_prefill(st, fs->q, ly.kc, ly.vc, attn, offset, S, mp->H, hd, mp->ctx, scale, streamed, cu));
         const vk::GemmNorm ffn_norm{ly.ffn_norm, xn, mp->eps, streamed};
         charge(ctx, fs, NS_WO, l);
         if (streamed)

@@ -5,7 +5,8 @@
 // p_j = fp16(exp(s_j - M) / L) there and 0 past it; out = fp16(sum_j p_j v_j). When kv == hd the reference reads the
 // V slice as [N, K] and the product becomes out[n] = fp16(sum_k p_k V[n][k]) (src/core/vkllm_op_matmul.c:14-24).
 //
-// A workgroup of 4 waves takes 64 query rows of one head; wave w owns rows [16 w, 16 w + 16), so every row's
+// A group of 4 waves takes 64 query rows of one head (a workgroup has one or two groups on the same rows, each with every
+// other key block); wave w owns rows [16 w, 16 w + 16), so every row's
 // statistics stay inside one wave. Key blocks of 64 positions go through two LDS buffers (K as [key][dim], V as
 // [dim][key]), shared by the 4 waves, with each block's global loads requested two blocks ahead (the kernel is
 // bound by that latency, not by the matrix pipe). Products use v_mfma_f32_16x16x32_f16 in the transposed orientation:
@@ -67,9 +68,11 @@ __device__ __forceinline__ float row4_sum(float v)
     return v + __shfl_xor(v, 32);
 }
 
-// ONE: kv <= 2 key blocks, computed in one pass (below); otherwise the two passes
-template <int HD, bool ONE>
-__global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *q, const uint16_t *kc,
+// ONE: kv <= 2 key blocks, computed in one pass (below); otherwise the two passes. G groups of 4 waves share the rows:
+// group g takes the key blocks g, g + G, ... through LDS buffers of its own, and the groups' statistics (after pass 1)
+// and sums (after pass 2) are merged through LDS.
+template <int HD, bool ONE, int G>
+__global__ __launch_bounds__(256 * G) void attn_prefill_mfma_kernel(const uint16_t *q, const uint16_t *kc,
                                                                 const uint16_t *vc, uint16_t *out, uint32_t offset,
                                                                 uint32_t S, uint32_t H, uint32_t ctx, float scale,
                                                                 bool xt)
@@ -83,7 +86,12 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
     constexpr int VT = HD * (kPfKeys / 8) / 256; // transposed rule: (row, key chunk) vectors per thread
     constexpr int VR = 2 * VP > VT ? 2 * VP : VT; // V registers per set (either layout: 2 VP == VT here)
     // two buffers each of the K tile ([key][dim]) and the V tile ([dim][key]); K buffers first
-    extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds[];
+    static_assert(G == 1 || !ONE, "the one-pass form has one group");
+    extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds_all[];
+    const uint32_t grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    uint16_t *const pf_lds = pf_lds_all + grp * (2 * (kPfKeys * KROW + HD * VROW));
+    // first position of this group's block i
+    auto at = [&](uint32_t i) { return (G * i + grp) * kPfKeys; };
     auto Kt = [&](int b) { return pf_lds + b * (kPfKeys * KROW); };
     auto Vt = [&](int b) { return pf_lds + 2 * kPfKeys * KROW + b * (HD * VROW); };
     // The V tile is read as 8-byte units (4 keys) by 16 lanes of 16 consecutive rows, and rows 8 apart fall on the
@@ -91,7 +99,7 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
     // once. Every access below has a lane-constant swizzle bit, folded into a per-lane column offset.
 
     const uint32_t D = H * HD, h = blockIdx.x;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q4 = lane >> 4, c16 = lane & 15;
+    const uint32_t tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, q4 = lane >> 4, c16 = lane & 15; // in the group
     // heads vary fastest and row blocks run last to first: the workgroups with the most causal work start first, and
     // a head's workgroups are dealt to one XCD (blocks go to the 8 XCDs round robin) when H is a multiple of 8
     const uint32_t row0 = (gridDim.y - 1 - blockIdx.y) * kPfRows;
@@ -135,8 +143,8 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
             }
         }
     };
-    load_v(S0{}, 0);
-    load_v(S1{}, kPfKeys);
+    load_v(S0{}, at(0));
+    load_v(S1{}, at(1));
 
     // Blocks stream through two register sets and the two LDS buffers: while block b is computed from buffer
     // b % 2, set b % 2 loads block b + 2 and set (b + 1) % 2 (block b + 1, requested a block earlier) is stored to
@@ -327,18 +335,19 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
     }
     float m = -FLT_MAX, l = 0.f;
     const uint32_t last = offset + min(row0 + kPfRows, S) - 1; // the workgroup's last position
-    const uint32_t nb1 = last / kPfKeys + 1;
+    // blocks of each group (the last one of the later group may lie past the last position: its steps only keep pace)
+    const uint32_t nb1 = (last / kPfKeys + G) / G;
     // nb1 <= 2: pass 1 leaves K blocks 0 and 1 in LDS buffers 0 and 1, where pass 2 reads them; otherwise pass
     // 1's last step requests them again (both register sets are free by then)
     const bool reuse_k = nb1 <= 2;
     auto step1 = [&](auto ld, auto cur, auto nxt, int buf, uint32_t jb) {
         if constexpr (decltype(ld)::value >= 1)
-            load_k(cur, jb + 2 * kPfKeys);
+            load_k(cur, jb + 2 * G * kPfKeys);
         if constexpr (decltype(ld)::value < 0)
             if (!reuse_k)
             {
-                load_k(S0{}, 0);
-                load_k(S1{}, kPfKeys);
+                load_k(S0{}, at(0));
+                load_k(S1{}, at(1));
             }
         f32x4a st[4];
         scores(buf, st);
@@ -386,25 +395,41 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
     using St = std::integral_constant<int, 0>;
     using Nn = std::integral_constant<int, -1>;
     const uint32_t nb1e = (nb1 + 1) & ~1u;
-    load_k(S0{}, 0);
-    load_k(S1{}, kPfKeys);
+    load_k(S0{}, at(0));
+    load_k(S1{}, at(1));
     store_k(S0{}, 0);
     __syncthreads();
     uint32_t blk = 0;
     for (; blk + 2 < nb1e; blk += 2)
     {
-        step1(Ld{}, S0{}, S1{}, 0, blk * kPfKeys);
-        step1(Ld{}, S1{}, S0{}, 1, (blk + 1) * kPfKeys);
+        step1(Ld{}, S0{}, S1{}, 0, at(blk));
+        step1(Ld{}, S1{}, S0{}, 1, at(blk + 1));
     }
     if (blk + 1 < nb1)
     {
-        step1(St{}, S0{}, S1{}, 0, blk * kPfKeys);
-        step1(Nn{}, S1{}, S0{}, 1, (blk + 1) * kPfKeys);
+        step1(St{}, S0{}, S1{}, 0, at(blk));
+        step1(Nn{}, S1{}, S0{}, 1, at(blk + 1));
     }
     else
-        step1(Nn{}, S0{}, S1{}, 0, blk * kPfKeys);
+        step1(Nn{}, S0{}, S1{}, 0, at(blk));
     __syncthreads(); // the last block's LDS reads are done before pass 2 stores into that buffer
-    const float M = m, L = row4_sum(l), inv_l = 1.0f / L, nM = -M * kLog2e;
+    float L = row4_sum(l);
+    if constexpr (G == 2)
+    {
+        // each group's max and sum of its keys, per row (a group without a live key for the row adds nothing)
+        __shared__ float sm[2][kPfRows], sl[2][kPfRows];
+        const uint32_t r = wave * 16 + c16;
+        if (q4 == 0)
+        {
+            sm[grp][r] = m;
+            sl[grp][r] = L;
+        }
+        __syncthreads();
+        const float m0 = sm[0][r], m1 = sm[1][r];
+        m = fmaxf(m0, m1);
+        L = sl[0][r] * pf_exp2((m0 - m) * kLog2e) + sl[1][r] * pf_exp2((m1 - m) * kLog2e);
+    }
+    const float M = m, inv_l = 1.0f / L, nM = -M * kLog2e;
 
     // ---- pass 2: probabilities and P.V over the blocks at or before the workgroup's last row
     const uint32_t nb2 = nb1;
@@ -444,12 +469,8 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
         }
     };
     const uint32_t vcol = 4 * (q4 ^ ((c16 >> 3) & 1u));
-    auto step2 = [&](auto ld, auto cur, auto nxt, int buf, uint32_t jb) {
-        if constexpr (decltype(ld)::value >= 1)
-        {
-            load_k(cur, jb + 2 * kPfKeys);
-            load_v(cur, jb + 2 * kPfKeys);
-        }
+    // the block's probabilities and P.V
+    auto pv = [&](int buf, uint32_t jb) {
         f32x4a st[4];
         scores(buf, st);
         _Float16 ph[4][4];
@@ -483,9 +504,18 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
                 o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pb, o[d], 0, 0, 0);
             }
         }
+    };
+    auto step2 = [&](auto ld, auto cur, auto nxt, int buf, uint32_t jb) {
+        if constexpr (decltype(ld)::value >= 1)
+        {
+            load_k(cur, jb + 2 * G * kPfKeys);
+            load_v(cur, jb + 2 * G * kPfKeys);
+        }
+        if (G == 1 || jb <= last)
+            pv(buf, jb);
         if constexpr (decltype(ld)::value >= 0)
         {
-            if (!reuse_k) // nb2 <= nb1, so with reuse_k this is block 1, already in buffer 1
+            if (!reuse_k) // nb2 == nb1, so with reuse_k this is block 1, already in buffer 1
                 store_k(nxt, buf ^ 1);
             store_v(nxt, buf ^ 1);
             __syncthreads();
@@ -499,16 +529,34 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const uint16_t *
     __syncthreads();
     for (blk = 0; blk + 2 < nb2e; blk += 2)
     {
-        step2(Ld{}, S0{}, S1{}, 0, blk * kPfKeys);
-        step2(Ld{}, S1{}, S0{}, 1, (blk + 1) * kPfKeys);
+        step2(Ld{}, S0{}, S1{}, 0, at(blk));
+        step2(Ld{}, S1{}, S0{}, 1, at(blk + 1));
     }
     if (blk + 1 < nb2)
     {
-        step2(St{}, S0{}, S1{}, 0, blk * kPfKeys);
-        step2(Nn{}, S1{}, S0{}, 1, (blk + 1) * kPfKeys);
+        step2(St{}, S0{}, S1{}, 0, at(blk));
+        step2(Nn{}, S1{}, S0{}, 1, at(blk + 1));
     }
     else
-        step2(Nn{}, S0{}, S1{}, 0, blk * kPfKeys);
+        step2(Nn{}, S0{}, S1{}, 0, at(blk));
+    if constexpr (G == 2)
+    {
+        // the groups' sums, group 1's through LDS (the tiles are free): 16 bytes per lane and output block
+        __syncthreads();
+        f32x4a *ex = (f32x4a *)pf_lds_all + tid;
+        if (grp == 1)
+        {
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+                ex[256 * d] = o[d];
+        }
+        __syncthreads();
+        if (grp == 1)
+            return;
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+            o[d] += ex[256 * d];
+    }
     // O^T accumulators: o[d][e] = out[row c16][dim 16 d + 4 q4 + e]
     const uint32_t row = row0 + wave * 16 + c16;
     if (row < S)
@@ -533,17 +581,17 @@ template <int HD> constexpr size_t pf_lds_bytes()
     return (size_t)2 * (kPfKeys * pf_krow<HD>() + HD * (kPfKeys + 8)) * sizeof(uint16_t);
 }
 
-template <int HD, bool ONE>
+template <int HD, bool ONE, int G>
 static hipError_t launch_pf_hd(hipStream_t st, dim3 grid, const uint16_t *q, const uint16_t *kc, const uint16_t *vc,
                                uint16_t *out, uint32_t offset, uint32_t S, uint32_t H, uint32_t ctx, float scale,
                                bool xt)
 {
     static uint64_t attr_devs = 0; // devices on which the LDS limit is raised for this kernel
-    constexpr size_t lds = pf_lds_bytes<HD>();
-    hipError_t e = lds_attr_once((const void *)attn_prefill_mfma_kernel<HD, ONE>, lds, attr_devs);
+    constexpr size_t lds = G * pf_lds_bytes<HD>();
+    hipError_t e = lds_attr_once((const void *)attn_prefill_mfma_kernel<HD, ONE, G>, lds, attr_devs);
     if (e != hipSuccess)
         return e;
-    attn_prefill_mfma_kernel<HD, ONE><<<grid, 256, lds, st>>>(q, kc, vc, out, offset, S, H, ctx, scale, xt);
+    attn_prefill_mfma_kernel<HD, ONE, G><<<grid, 256 * G, lds, st>>>(q, kc, vc, out, offset, S, H, ctx, scale, xt);
     return hipGetLastError();
 }
 
@@ -554,19 +602,25 @@ bool attn_prefill_mfma_ok(uint32_t hd)
 
 hipError_t launch_attn_prefill_mfma(hipStream_t st, const uint16_t *q, const uint16_t *kc, const uint16_t *vc,
                                     uint16_t *out, uint32_t offset, uint32_t S, uint32_t H, uint32_t hd, uint32_t ctx,
-                                    float scale, bool xt)
+                                    float scale, bool xt, int cu_count)
 {
     if (S == 0 || offset + S > ctx || !attn_prefill_mfma_ok(hd) || (xt && S > 128))
         return hipErrorInvalidValue;
     const dim3 grid(H, (S + kPfRows - 1) / kPfRows);
-    // a step whose kv fits two key blocks takes the one-pass form (its own instantiation, so the two-pass kernel's
-    // code and registers are those it has without it)
+    // a step whose kv fits two key blocks takes the one-pass form
     const bool one = offset + S <= 2 * kPfKeys;
-    if (hd == 128)
-        return one ? launch_pf_hd<128, true>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt)
-                   : launch_pf_hd<128, false>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt);
-    return one ? launch_pf_hd<64, true>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt)
-               : launch_pf_hd<64, false>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt);
+    // two groups of waves halve the chain of key blocks that a workgroup walks but take the LDS of two workgroups: for
+    // grids that leave no second workgroup for a CU. us a layer, one / two groups (7B widths unless said): 160 workgroups
+    // (301 tokens behind 700) 44.1 / 34.9, 32 (5 tokens behind 900) 38.8 / 31.6, 320 (600 tokens) 32.8 / 26.9, 512 (1024
+    // tokens) 52.6 / 51.0; 13B widths, 840 (1300 tokens behind 500) 151 / 168, 1280 (2048 tokens) 168 / 196
+    const bool two = (uint64_t)grid.x * grid.y < 2ull * (cu_count > 0 ? cu_count : 256);
+    auto go = [&](auto hd_tag) {
+        constexpr int HD = decltype(hd_tag)::value;
+        return one   ? launch_pf_hd<HD, true, 1>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt)
+               : two ? launch_pf_hd<HD, false, 2>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt)
+                     : launch_pf_hd<HD, false, 1>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt);
+    };
+    return hd == 128 ? go(std::integral_constant<int, 128>{}) : go(std::integral_constant<int, 64>{});
 }
 
 } // namespace vk

@@ -1093,12 +1093,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const uint16_t *q, co
 
 hipError_t launch_attn_prefill(hipStream_t st, const uint16_t *q, const uint16_t *kc, const uint16_t *vc,
                                uint16_t *out, uint32_t offset, uint32_t S, uint32_t H, uint32_t hd, uint32_t ctx,
-                               float scale, bool xt)
+                               float scale, bool xt, int cu_count)
 {
     if (hd % 8 != 0 || hd > 256)
         return hipErrorInvalidValue;
     if (attn_prefill_mfma_ok(hd))
-        return launch_attn_prefill_mfma(st, q, kc, vc, out, offset, S, H, hd, ctx, scale, xt);
+        return launch_attn_prefill_mfma(st, q, kc, vc, out, offset, S, H, hd, ctx, scale, xt, cu_count);
     if (xt) // fragment-ordered output from the MFMA kernel only
         return hipErrorInvalidValue;
     const size_t lds = (size_t)(offset + S) * sizeof(float);

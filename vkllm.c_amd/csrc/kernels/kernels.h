@@ -238,10 +238,10 @@ bool attn_prefill_mfma_ok(uint32_t hd);
 // with xt, out is fragment-ordered (xt_vec; S <= 128)
 hipError_t launch_attn_prefill_mfma(hipStream_t st, const uint16_t *q, const uint16_t *kc, const uint16_t *vc,
                                     uint16_t *out, uint32_t offset, uint32_t S, uint32_t H, uint32_t hd, uint32_t ctx,
-                                    float scale, bool xt = false);
+                                    float scale, bool xt = false, int cu_count = 0);
 hipError_t launch_attn_prefill(hipStream_t st, const uint16_t *q, const uint16_t *kc, const uint16_t *vc,
                                uint16_t *out, uint32_t offset, uint32_t S, uint32_t H, uint32_t hd, uint32_t ctx,
-                               float scale, bool xt = false);
+                               float scale, bool xt = false, int cu_count = 0);
 // qkv [S, 3D] -> RoPE'd q [S, D]; RoPE'd k and v into the caches at rows offset..offset+S-1
 hipError_t launch_rope_kv(hipStream_t st, const uint16_t *qkv, uint16_t *q, uint16_t *kc, uint16_t *vc,
                           const float *freqs, uint32_t offset, uint32_t S, uint32_t D, uint32_t hd, uint32_t ctx);
