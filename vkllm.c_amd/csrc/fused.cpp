@@ -40,6 +40,7 @@ struct FusedState
     uint32_t cap_S = 0; // rows the activation buffers hold
     uint16_t *h = nullptr, *xn = nullptr, *qkv = nullptr, *q = nullptr, *attn = nullptr, *act = nullptr,
              *ug = nullptr, *logits = nullptr;
+    float2 *step_cs = nullptr;   // a single-token step's RoPE rotations [hd / 2], shared by its layers
     uint32_t *ids = nullptr;
     float *rope_cs = nullptr;    // a prompt step's RoPE angles [S][hd / 2][2], shared by its layers
     vk::Step *step = nullptr;    // device
@@ -294,6 +295,8 @@ void fused_model_release(vkllm_context *ctx, vkllm_models_llama2 *model)
     free_buffers(fs);
     if (fs->step)
         (void)hipFree(fs->step);
+    if (fs->step_cs)
+        (void)hipFree(fs->step_cs);
     if (fs->freqs)
         (void)hipFree(fs->freqs);
     free_stream_tiles(fs);
@@ -414,6 +417,8 @@ static vkllm_err_t ensure_state(vkllm_context *ctx, ModelPriv *mp, uint32_t S)
             HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         const char *la = getenv("VKLLM_LAUNCH_AHEAD");
         fs->ahead_enabled = !(la && *la == '0');
+        HIP_TRY(hipMalloc(&fs->step_cs, sizeof(float2) * (mp->hd / 2 + 1)));
+        HIP_TRY(hipMemset(fs->step_cs, 0, sizeof(float2) * (mp->hd / 2 + 1)));
         HIP_TRY(hipMalloc(&fs->freqs, sizeof(float) * (mp->hd / 2 + 1)));
         HIP_TRY(hipMemcpyAsync(fs->freqs, mp->rope_freqs.data(), sizeof(float) * mp->hd / 2, hipMemcpyHostToDevice,
                                ctx->device->stream));
@@ -551,7 +556,7 @@ static hipError_t launch_decode_kernel(vkllm_context *ctx, ModelPriv *mp, Kernel
     {
     case KID_F_EMBED:
         return vk::launch_embed_decode(st, fs->dio, fs->step, mp->embd, resid_out ? resid_out : fs->h, V, D,
-                                       mp->pad_id, fs->slot_ids + (1 - fs->slot));
+                                       mp->pad_id, fs->slot_ids + (1 - fs->slot), fs->step_cs, fs->freqs, mp->hd);
     case KID_F_QKV:
         // RMSNorm(h) -> [Wq;Wk;Wv] -> RoPE(q, k); q to fs->q, k and v into the caches at the step's position
         g.x = fs->h;
@@ -564,6 +569,7 @@ static hipError_t launch_decode_kernel(vkllm_context *ctx, ModelPriv *mp, Kernel
         g.vc = ly.vc;
         g.step = fs->step;
         g.freqs = fs->freqs;
+        g.cs = fs->step_cs;
         g.D = D;
         g.hd = hd;
         g.ctx = mp->ctx;
@@ -767,7 +773,7 @@ static vkllm_err_t enqueue_decode(vkllm_context *ctx, ModelPriv *mp, uint32_t va
         FusedState *fs = mp->fs;
         KTRY(ctx, KID_F_EMBED,
              vk::launch_embed_decode(ctx->device->stream, fs->dio, fs->step, mp->embd, fs->p_hs, mp->V, mp->D,
-                                     mp->pad_id, fs->slot_ids + (1 - fs->slot)));
+                                     mp->pad_id, fs->slot_ids + (1 - fs->slot), fs->step_cs, fs->freqs, mp->hd));
         const hipError_t e = launch_persist(ctx, mp);
         fs->p_variant[variant] = e == hipSuccess;
         if (e == hipSuccess)
@@ -1351,7 +1357,7 @@ extern "C" vkllm_err_t vkllm_hip_model_time_kernel(struct vkllm_context *ctx, st
     };
     if (persist) // the last step's embedding row and position again (a step launched ahead wrote its own)
         HIP_TRY(vk::launch_embed_decode(st, fs->dio, fs->step, mp->embd, fs->p_hs, mp->V, mp->D, mp->pad_id,
-                                        fs->slot_ids + (1 - fs->slot)));
+                                        fs->slot_ids + (1 - fs->slot), fs->step_cs, fs->freqs, mp->hd));
     // one untimed launch so the first timed one does not pay for code loading
     HIP_TRY(launch(0));
     hipEvent_t ev[2];

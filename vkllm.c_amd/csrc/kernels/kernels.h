@@ -63,9 +63,10 @@ struct DecodeIo
     uint32_t token_dev; // nonzero: the step's token is the device-side arg max of the step before (launch-ahead)
 };
 // single-token step: step = {io->offset, 1}, h = embd[token] (ids >= V read row unk), where token is io->token, or
-// *prev_id when io->token_dev is set
+// *prev_id when io->token_dev is set; cs[w] = (cos, sin) of io->offset / freqs[w], w < hd / 2 (hd <= 256)
 hipError_t launch_embed_decode(hipStream_t st, const DecodeIo *io, Step *step, const uint16_t *embd, uint16_t *h,
-                               uint32_t V, uint32_t D, uint32_t unk, const uint32_t *prev_id);
+                               uint32_t V, uint32_t D, uint32_t unk, const uint32_t *prev_id, float2 *cs,
+                               const float *freqs, uint32_t hd);
 // *step = now, and h[s] = embd[toks[s]] (ids >= V read row unk), s < now.S; D % 8 == 0; toks in pinned or device memory
 hipError_t launch_embed_rows(hipStream_t st, const uint32_t *toks, const Step &now, Step *step, const uint16_t *embd,
                              uint16_t *h, uint32_t V, uint32_t D, uint32_t unk);
@@ -112,7 +113,8 @@ struct GemvArgs
     // EPI_QKV
     uint16_t *kc, *vc;      // layer caches [H, ctx, hd]
     const Step *step;
-    const float *freqs;     // base^(2w/hd), w < hd/2
+    const float *freqs;     // base^(2w/hd), w < hd/2 (the fallback kernel)
+    const float2 *cs;       // the position's rotations (cos, sin), w < hd/2, from launch_embed_decode
     uint32_t D, hd, ctx;
     // EPI_QKV_ATTN
     uint16_t *attn_out;     // [H, hd]
