@@ -69,3 +69,24 @@ def test_matmul_batched(ctx, vk, case, pad):
         atol = 1.1 * atol + 2.0 ** -21 * np.abs(want)
         want = want / (1.0 + np.exp(-want))
     assert_fp16_close(got, want.astype(np.float16), what=str(case), atol=atol + 2.0 ** -24)
+
+
+def test_matmul_rows_past_the_ring_kernels_offsets(ctx, vk):
+    """Rows of more than 2^22 elements (the LDS-ring tile kernel's byte offsets are 32-bit): +-1 at a few places, the
+    last ones included, so the sums are whole numbers and exact."""
+    M, N, K = 2, 8, (1 << 22) + 64
+    print(f"[matmul] {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(3)
+    at = np.unique(np.concatenate([rng.integers(0, K, 500), [0, (1 << 22) - 1, 1 << 22, K - 1]]))
+    a, b = np.zeros((1, 1, M, K), np.float16), np.zeros((1, 1, N, K), np.float16)
+    a[..., at], b[..., at] = (rng.choice([-1.0, 1.0], (1, 1, n, at.size)) for n in (M, N))
+    ta, tb = ctx.tensor_from(a), ctx.tensor_from(b)
+    out = ctx.tensor([1, 1, M, N], vk.F16, op=vk.OP_MATMUL, srcs=[ta, tb], params=vk.MatmulParams(1.0, 0))
+    try:
+        vk.check("matmul", ctx.run_op("matmul", out))
+        got = ctx.download(out).reshape(M, N)
+    finally:
+        for t in (out, ta, tb):
+            ctx.free(t)
+    want = a[0, 0][:, at].astype(np.float64) @ b[0, 0][:, at].astype(np.float64).T
+    assert np.array_equal(got.astype(np.float64), want)

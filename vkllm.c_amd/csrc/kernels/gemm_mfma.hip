@@ -929,16 +929,17 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
 {
     const uint32_t cus = cu_count > 0 ? (uint32_t)cu_count : 256;
     if constexpr (EPI == GEMM_QKV_ROPE)
-        if (!rope || K % kBK != 0 || rope->D % 64 != 0 || rope->hd < 32 || (rope->hd & (rope->hd - 1)) != 0 ||
+        if (!rope || K % kBK != 0 || K > kGemm32MaxK || rope->D % 64 != 0 || rope->hd < 32 || (rope->hd & (rope->hd - 1)) != 0 ||
             N != 3 * rope->D || !rope->cs)
             return hipErrorInvalidValue;
     if ((uint64_t)N * K >= (1ull << 32)) // B row offsets are 32-bit
         return hipErrorInvalidValue;
     if constexpr (is_dual(EPI))
-        if (K % kBK != 0 || N % 64 != 0 || N != (2 * split + 63) / 64 * 64 || split % 8 != 0 || !B.p2 || ldc % 8 != 0 ||
+        if (K % kBK != 0 || K > kGemm32MaxK || N % 64 != 0 || N != (2 * split + 63) / 64 * 64 || split % 8 != 0 || !B.p2 || ldc % 8 != 0 ||
             (uintptr_t)C % 16 != 0)
             return hipErrorInvalidValue;
-    if (K % kBK == 0)
+    // (gemm32_kernel's copies address a tile's rows by 32-bit byte offsets; longer rows take gemm_kernel)
+    if (K % kBK == 0 && K <= kGemm32MaxK)
     {
         const TileChoice c = pick_tile(M, N, K, cus, work_elems, EPI == GEMM_RESID && norm);
         const uint32_t kchunk = ((K + c.splits - 1) / c.splits + kBK - 1) / kBK * kBK, splits = (K + kchunk - 1) / kchunk;

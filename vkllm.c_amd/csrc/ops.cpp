@@ -669,7 +669,7 @@ static FfnPath ffn_path(const vk::TView &x, const vk::TView &wu, const vk::TView
         return FfnPath::GENERIC;
     if (rows == 1 && K % 8 == 0 && K > 0 && K <= 8 * 64 * 22)
         return FfnPath::ROW;
-    if (K > 0 && K % 64 == 0 && F % 8 == 0 && 2ull * F * K < (1ull << 32) - 64ull * K)
+    if (K > 0 && K % 64 == 0 && K <= vk::kGemm32MaxK && F % 8 == 0 && 2ull * F * K < (1ull << 32) - 64ull * K)
         return FfnPath::TILES;
     return rows <= 256 && vk::gemm_small_ok((uint32_t)rows, F, K) ? FfnPath::SMALL : FfnPath::GENERIC;
 }
