@@ -100,7 +100,9 @@ extern vkllm_err_t vkllm_hip_model_last_logits(struct vkllm_context *context, st
  * vkllm_graph_post_run -> vkllm_tensor_invalid_cache -> read the last id -> vkllm_graph_free.
  * ids[i] receives step i's last arg-max id, step_ns[i] (optional) the step's wall time, and phase_ns[4] (optional)
  * the wall time summed over steps 1.. of: tensor_new + graph_new + build_graph; graph_init + upload;
- * graph_run + post_run; invalid_cache + read + graph_free. The last of 4 or more steps launches no step ahead. */
+ * graph_run + post_run; invalid_cache + read + graph_free.
+ * The call's last step, like any single-token step, launches the next one ahead, for a caller that goes on where the
+ * call ends; once the steps launched behind two calls in a row went unused, it does not, until a call goes on. */
 extern vkllm_err_t vkllm_hip_token_loop(struct vkllm_context *context, struct vkllm_models_llama2 *model,
                                         const uint32_t *prompt, uint32_t prompt_len, uint32_t offset0,
                                         uint32_t n_steps, uint32_t *ids, uint64_t *step_ns, uint64_t *phase_ns);

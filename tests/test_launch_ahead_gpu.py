@@ -4,7 +4,10 @@ p + 1 (the reference driver's greedy loop, tests/vkllm_test_infer_gguf.c:255-269
 discards it. These tests drive both paths against the oracle, which simply runs the calls it is given, and check that
 the switch VKLLM_LAUNCH_AHEAD=0 changes no result.
 """
+import ctypes
+
 import numpy as np
+import pyvkllm
 import pytest
 
 from helpers import fp16_ulp
@@ -101,6 +104,53 @@ def test_switch_changes_no_result(ctx, vk, oracle, monkeypatch):
             print(f"step {i}: oracle margin {top2[1] - top2[0]:.4f}; streams compared up to it")
             break
         assert a == b, f"step {i}: id {a} vs oracle {b} at margin {top2[1] - top2[0]:.4f}"
+
+
+def _cache_row_written(ctx, model, pos):
+    """Whether the keys of position `pos` in layer 0 hold anything: a step at that position, asked for or ahead, ran."""
+    ctx.sync()
+    kcaches = ctypes.cast(model.m.weights.kvcache, ctypes.POINTER(ctypes.POINTER(pyvkllm.ArrayTensor))).contents
+    k = ctx.download(kcaches.contents.data[0]).reshape(SHAPE["n_head"], SHAPE["ctx"], -1)
+    return bool(np.any(k[:, pos] != 0))
+
+
+@pytest.mark.parametrize("steps", [1, 3, 4, 6])
+def test_token_loops_that_go_on_keep_the_step_ahead(ctx, vk, oracle, steps):
+    """One sequence generated in calls of `steps` steps: every call's last step has launched the next one ahead (its
+    cache row is written when the call's work is done), whatever the calls' length."""
+    cfg, ref, model = _pair(oracle, vk, ctx, seed=89)
+    try:
+        prompt = oracle.prompt_tokens(90, 8, cfg.vocab)
+        want = ref.token_loop(prompt, 1 + 6 * steps)[0].tolist()
+        got = [int(model.step(prompt, 0)[-1])]
+        for call in range(6):
+            pos = len(prompt) + len(got) - 1
+            got += model.loop(np.array(got[-1:], np.uint32), steps, pos)[0].tolist()
+            assert _cache_row_written(ctx, model, pos + steps), f"call {call} of {steps} steps launched nothing ahead"
+        assert got == want
+    finally:
+        ref.close()
+        model.close()
+
+
+def test_token_loops_that_end_drop_the_step_ahead(ctx, vk, oracle):
+    """Calls that nobody goes on from: the third and later launch no step behind their last one, until a call goes on
+    where the one before ended. Each call is one position longer than those before, so its next row is still zero."""
+    cfg, ref, model = _pair(oracle, vk, ctx, seed=91)
+    try:
+        prompt = oracle.prompt_tokens(92, 8, cfg.vocab)
+        first = int(model.step(prompt, 0)[-1])
+        for steps, ahead in ((4, True), (6, True), (8, False), (9, False)):
+            ids = model.loop(np.array([first], np.uint32), steps, 8)[0]
+            assert _cache_row_written(ctx, model, 8 + steps) == ahead, f"call of {steps} steps"
+        pos = 8 + steps
+        ids = model.loop(ids[-1:], 4, pos)[0]  # goes on
+        assert _cache_row_written(ctx, model, pos + 4)
+        want = ref.token_loop(prompt, 1 + steps + 4)[0].tolist()
+        assert ids.tolist() == want[1 + steps:]
+    finally:
+        ref.close()
+        model.close()
 
 
 def test_two_models_interleaved(ctx, vk, oracle):

@@ -40,11 +40,7 @@ extern "C" vkllm_err_t vkllm_hip_token_loop(struct vkllm_context *context, struc
         }
         // build_graph adopts input_toks into the graph and frees the graph itself on failure
         _CHECK(vkllm_models_llama2_build_graph(context, model, input_toks, graph, offset));
-        // The loop knows its last step: launching the next one ahead would run a whole token that the next call, a
-        // prompt or another sequence as a rule, throws away (16 steps of a 4-layer 7B-wide model 6098 -> 5757 us). A
-        // caller who goes on in calls of a few steps pays 16 us a call instead (the host's work and the launch, no
-        // longer hidden), so calls of fewer than 4 steps keep it.
-        if (i + 1 == n_steps && n_steps >= 4 && graph->plan)
+        if (i + 1 == n_steps && graph->plan)
             fused_plan_last_step(graph->plan);
         const uint64_t t1 = now_ns();
         rc = vkllm_graph_init(context, graph);

@@ -10,6 +10,7 @@
 //           the residual add -> RMSNorm -> [up;gate] GEMM with SiLU on the gate half -> up*gate -> Wd GEMM with
 //           the residual add; then RMSNorm -> logits GEMM for all S rows -> arg max per row.
 // Either way the S arg-max ids land in the mapped output tensor, as the reference's ARG_MAX node leaves them.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -28,8 +29,14 @@ struct FusedPlan
     uint32_t offset;
     uint32_t S;
     bool ran = false; // fused_plan_run enqueued (and completed) the step
-    bool last = false; // the caller says that no step at the next position follows
+    bool last = false; // the last step of a token loop's call
 };
+
+// A token loop's last step launches the next one ahead until the steps launched behind this many calls in a row went
+// unused. A step that nobody takes costs a whole token (the next call's first step waits for it: 340 us at 4 layers of
+// the 7B widths, 115 us on the tiny decoder), one that is missing where a caller goes on costs the host's work and the
+// launch it would have hidden (16 us). With two, a caller that generates in several calls a sequence never turns it off.
+constexpr uint32_t kLoopUnusedMax = 2;
 
 // Short-cache decode steps are captured per bucket of kSmallBucket cache positions: a bucket's launches bound their
 // LDS and the keys and V rows they request before the position is known by the bucket's end.
@@ -67,6 +74,10 @@ struct FusedState
     bool ahead_live = false;
     int ahead_slot = 0;
     uint32_t ahead_offset = 0, ahead_token = 0; // the step launched ahead: its position, and its token once known
+    // where the last token loop ended (the position and token of a call that goes on), until the next step shows
+    // whether the caller does, and the calls in a row so far that nobody went on from
+    bool loop_ended = false;
+    uint32_t loop_offset = 0, loop_token = 0, loop_unused = 0;
     // the last completed single-token step (what vkllm_hip_model_last_logits and the timing replays refer to)
     int done_slot = 0;
     uint32_t done_offset = 0, done_token = 0;
@@ -1159,6 +1170,12 @@ vkllm_err_t fused_plan_run(vkllm_context *ctx, vkllm_graph *graph)
     // the step's ids are in the mapped input tensor's host mirror (written by vkllm_commands_upload)
     const uint32_t *toks = (const uint32_t *)p->input_toks->data.host;
     vkllm_tensor *out = graph->output_node;
+    if (fs->loop_ended)
+    {
+        const bool goes_on = S == 1 && p->offset == fs->loop_offset && toks[0] == fs->loop_token;
+        fs->loop_unused = goes_on ? 0 : std::min(fs->loop_unused + 1, kLoopUnusedMax);
+        fs->loop_ended = false;
+    }
     if (S == 1)
     {
         // position and token go through the slot's pinned block that the step's first kernel reads; the arg max
@@ -1183,7 +1200,7 @@ vkllm_err_t fused_plan_run(vkllm_context *ctx, vkllm_graph *graph)
             HIP_TRY(hipEventRecord(fs->slot_done[slot], st));
         }
         fs->ahead_live = false;
-        if (fs->ahead_enabled && !p->last && !direct && p->offset + 1 < mp->ctx)
+        if (fs->ahead_enabled && !(p->last && fs->loop_unused >= kLoopUnusedMax) && !direct && p->offset + 1 < mp->ctx)
         {
             // the step at p + 1 behind this one, its token this step's device-side arg max
             const int nx = 1 - slot;
@@ -1233,6 +1250,12 @@ vkllm_err_t fused_plan_run(vkllm_context *ctx, vkllm_graph *graph)
         fs->io_h[0] = id;
         if (fs->ahead_live)
             fs->ahead_token = id;
+        if (p->last && p->offset + 1 < mp->ctx)
+        {
+            fs->loop_ended = true;
+            fs->loop_offset = p->offset + 1;
+            fs->loop_token = id;
+        }
         fs->done_slot = slot;
         fs->done_offset = p->offset;
         fs->done_token = toks[0];

@@ -195,7 +195,8 @@ vkllm_err_t fused_plan_init(vkllm_context *ctx, vkllm_graph *graph);
 vkllm_err_t fused_plan_run(vkllm_context *ctx, vkllm_graph *graph);
 // true once the plan ran as fused kernels (which read none of the graph's node tensors)
 bool fused_plan_ran(const void *plan);
-// the plan's step, if it is a single-token one, launches no step ahead
+// the plan's step is the last of a token loop's call: whether it launches the next one ahead follows from what became
+// of the steps launched behind the calls before
 void fused_plan_last_step(void *plan);
 // drops a single-token step launched ahead for the plan's model (before node-by-node execution of its graph)
 vkllm_err_t fused_plan_discard_ahead(vkllm_context *ctx, vkllm_graph *graph);
