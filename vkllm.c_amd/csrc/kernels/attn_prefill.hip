@@ -1,7 +1,7 @@
 // Prefill attention on CDNA4 matrix cores: the S query rows of a step against the kv = offset + S cached positions
 // of each head (src/models/vkllm_llama2_layers.c:223-257 with src/shaders/vkllm_softmax.comp:42-96), keeping the
-// reference's rounding points: s_j = fp16(scale * q.k_j); M = a max over the row's scores; L = sum of exp(s_j - M)
-// over j <= the row's position;
+// reference's rounding points: s_j = fp16(scale * q.k_j); M = max over the WHOLE row (j < kv, later positions
+// included, as the softmax shader takes it); L = sum of exp(s_j - M) over j <= the row's position;
 // p_j = fp16(exp(s_j - M) / L) there and 0 past it; out = fp16(sum_j p_j v_j). When kv == hd the reference reads the
 // V slice as [N, K] and the product becomes out[n] = fp16(sum_k p_k V[n][k]) (src/core/vkllm_op_matmul.c:14-24).
 //
@@ -14,10 +14,9 @@
 //   O^T += V^T . P^T (A = the V tile read as [dim][key], B = the probabilities straight from the S^T
 //                     accumulators: the 32 keys of a K slice are ordered so that lane l's 8 slots are the 4 keys
 //                     of each of two 16-key score blocks that it holds)
-// Pass 1 walks the blocks at or before the workgroup's last row for M and L (an online sum, rescaled when the row max
-// grows). The softmax shader's max runs over the whole row, later positions included; exp(s - M) / L does not depend on
-// M but for the rounding of exp, so the later blocks are left out (13B widths, 2048 tokens: 210 -> 168 us a layer;
-// shorter prompts are bound by the chain of their last rows, which see every block). Pass 2 recomputes
+// Pass 1 walks all kv positions for M and L (an online sum, rescaled when the row max grows). The blocks past the
+// workgroup's last row count: exp(s - M) / L depends on M where a later score exceeds the row's own by more than the
+// exponent's range, and is then 0 / 0 as in the softmax shader. Pass 2 recomputes
 // the same scores (same instructions, same order, so the same fp16 values) for the blocks at or before the last
 // row's position and accumulates P.V. Pass 2's first two V blocks are requested at entry and its first two K blocks
 // in pass 1's last step (or, for kv <= 128, read from where pass 1 left them in LDS), so pass 2 starts without a
@@ -187,7 +186,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_mfma_kernel(const uint16
         }
     };
 
-    // ---- pass 1: row max over the blocks up to the workgroup's last row, sum of exp over the causal positions
+    // ---- pass 1: row max over all kv positions, sum of exp over the causal ones
     // The wave's rows span positions [pos_lo, pos_hi]: a block wholly before pos_lo (and inside kv) needs no masks,
     // and a block wholly after pos_hi adds nothing to the sums, only to the max.
     const uint32_t pos_lo = offset + min(row0 + wave * 16, S - 1), pos_hi = offset + min(row0 + wave * 16 + 15, S - 1);
@@ -335,8 +334,8 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_mfma_kernel(const uint16
     }
     float m = -FLT_MAX, l = 0.f;
     const uint32_t last = offset + min(row0 + kPfRows, S) - 1; // the workgroup's last position
-    // blocks of each group (the last one of the later group may lie past the last position: its steps only keep pace)
-    const uint32_t nb1 = (last / kPfKeys + G) / G;
+    // blocks of each group in the passes (the last one of the later group may lie past the end: its steps only keep pace)
+    const uint32_t nb1 = ((kv - 1) / kPfKeys + G) / G, nb2 = (last / kPfKeys + G) / G;
     // nb1 <= 2: pass 1 leaves K blocks 0 and 1 in LDS buffers 0 and 1, where pass 2 reads them; otherwise pass
     // 1's last step requests them again (both register sets are free by then)
     const bool reuse_k = nb1 <= 2;
@@ -427,12 +426,11 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_mfma_kernel(const uint16
         __syncthreads();
         const float m0 = sm[0][r], m1 = sm[1][r];
         m = fmaxf(m0, m1);
-        L = sl[0][r] * pf_exp2((m0 - m) * kLog2e) + sl[1][r] * pf_exp2((m1 - m) * kLog2e);
+        L = fmaf(sl[0][r], pf_exp2((m0 - m) * kLog2e), sl[1][r] * pf_exp2((m1 - m) * kLog2e));
     }
     const float M = m, inv_l = 1.0f / L, nM = -M * kLog2e;
 
     // ---- pass 2: probabilities and P.V over the blocks at or before the workgroup's last row
-    const uint32_t nb2 = nb1;
     f32x4a o[DB];
 #pragma unroll
     for (int d = 0; d < DB; ++d)
@@ -515,7 +513,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_mfma_kernel(const uint16
             pv(buf, jb);
         if constexpr (decltype(ld)::value >= 0)
         {
-            if (!reuse_k) // nb2 == nb1, so with reuse_k this is block 1, already in buffer 1
+            if (!reuse_k) // nb2 <= nb1, so with reuse_k this is block 1, already in buffer 1
                 store_k(nxt, buf ^ 1);
             store_v(nxt, buf ^ 1);
             __syncthreads();
@@ -610,10 +608,11 @@ hipError_t launch_attn_prefill_mfma(hipStream_t st, const uint16_t *q, const uin
     // a step whose kv fits two key blocks takes the one-pass form
     const bool one = offset + S <= 2 * kPfKeys;
     // two groups of waves halve the chain of key blocks that a workgroup walks but take the LDS of two workgroups: for
-    // grids that leave no second workgroup for a CU. us a layer, one / two groups (7B widths unless said): 160 workgroups
-    // (301 tokens behind 700) 44.1 / 34.9, 32 (5 tokens behind 900) 38.8 / 31.6, 320 (600 tokens) 32.8 / 26.9, 512 (1024
-    // tokens) 52.6 / 51.0; 13B widths, 840 (1300 tokens behind 500) 151 / 168, 1280 (2048 tokens) 168 / 196
-    const bool two = (uint64_t)grid.x * grid.y < 2ull * (cu_count > 0 ? cu_count : 256);
+    // grids of at most one workgroup a CU. us a layer, one / two groups, head size 128: 32 workgroups (5 tokens behind
+    // 900) 37.4 / 29.8, 160 (301 behind 700) 41.5 / 32.3, 256 (512 tokens) 22.7 / 19.0 and (512 behind 1500) 76.6 / 58.0;
+    // 280 (400 tokens, 40 heads) 21.3 / 24.3, 320 (600 tokens) 29.5 / 29.8, 512 (1024 tokens) 43.9 / 46.8, 1280 (2048
+    // tokens, 40 heads) 186 / 203
+    const bool two = (uint64_t)grid.x * grid.y <= (uint64_t)(cu_count > 0 ? cu_count : 256);
     auto go = [&](auto hd_tag) {
         constexpr int HD = decltype(hd_tag)::value;
         return one   ? launch_pf_hd<HD, true, 1>(st, grid, q, kc, vc, out, offset, S, H, ctx, scale, xt)
