@@ -152,3 +152,20 @@ def test_gemm_rejects_bad_arguments(ctx, vk):
     assert L.vkllm_hip_gemm(ctx.vp, PLAIN, p, q, p, 4, 4, 16, 4, 0, None, 0) == vk.ERR_ARGS  # B not 16-byte aligned
     assert L.vkllm_hip_gemm(ctx.vp, PLAIN, p, p, p, 4, 4, 16, 4, 0, q, 64) == vk.ERR_ARGS  # work not aligned
     assert L.vkllm_hip_gemm(ctx.vp, SWIGLU, p, p, q, 4, 128, 64, 64, 64, None, 0) == vk.ERR_ARGS  # C not aligned
+
+
+def test_swiglu_rows_past_the_32_bit_offsets(ctx, vk):
+    """SwiGLU over rows of more than 2^22 elements (a tile's rows then span more than 4 GB): +-1 at a few places of A and
+    B, the last ones and those past 2^22 included, so both sums are whole numbers. Rows of A in two tiles and past the
+    last one."""
+    M, F, K = 70, 32, (1 << 22) + 64
+    N = 2 * F
+    print(f"[gemm] SWIGLU {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(17)
+    at = np.unique(np.concatenate([rng.integers(0, K, 60), [0, (1 << 22) - 1, 1 << 22, K - 1]]))
+    a, b = np.zeros((M, K), np.float16), np.zeros((N, K), np.float16)
+    a[:, at], b[:, at] = (rng.choice([-1.0, 1.0], (n, at.size)) for n in (M, N))
+    got = run_gemm(ctx, vk, a, b, np.zeros((M, F), np.float16), SWIGLU, F, False).astype(np.float32)
+    ref = reference(a[:, at], b[:, at], None, SWIGLU, F)
+    # the sums are exact; silu and then the product may each land on the neighbouring fp16 value (2^-10 at most)
+    assert np.all(np.abs(got - ref) <= 2.0 ** -9 * np.abs(ref) + 2.0 ** -24)

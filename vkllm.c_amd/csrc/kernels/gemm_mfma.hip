@@ -262,9 +262,9 @@ template <int BM, int BN> constexpr int gemm_ring()
 }
 
 // n_base: product column of the kernel's column 0 (B rows and C columns are addressed from it; N counts the
-// kernel's columns). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
+// kernel's columns). WIDE: rows of any length, a tile's rows by 64-bit offsets (otherwise K <= kGemm32MaxK). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
 // blocks and `split` holds F.
-template <int BM, int BN, int EPI, bool SPLIT>
+template <int BM, int BN, int EPI, bool SPLIT, bool WIDE = false>
 __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                         const uint16_t *__restrict__ B2, uint16_t *C, float *work,
                                                         uint32_t M, uint32_t N, uint32_t K, uint32_t ldc,
@@ -296,7 +296,8 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
     const char *const Ap = (const char *)(A + (size_t)m0 * K + kb);
     // dual products: waves 0 and 1 copy the up rows of each block, waves 2 and 3 its gate rows
     const char *const Bp = (const char *)((is_dual(EPI) && wid >= 2 ? B2 : B) + (size_t)n_first * K + kb);
-    uint32_t voff[2][ND]; // byte offsets from those
+    using Off = std::conditional_t<WIDE, uint64_t, uint32_t>;
+    Off voff[2][ND]; // byte offsets from those
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -306,15 +307,19 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
             const int blk = i < NAI ? i + h * TM : i - NAI + h * TN;
             const uint32_t row = i < NAI ? min(32 * blk + r, M - 1 - m0)
                                          : min(is_dual(EPI) ? 16 * blk + r % 16 : 32 * blk + r, n_last - n_first);
-            voff[h][i] = row * K * 2 + ((lane ^ (r & 7)) & 7) * 16;
+            voff[h][i] = (Off)row * K * 2 + ((lane ^ (r & 7)) & 7) * 16;
         }
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)lds + wid * 1024;
     auto copy = [&](auto h_tag, int i, uint32_t slot, uint32_t kbyte) {
         constexpr int H = decltype(h_tag)::value;
         const char *base = (i < NAI ? Ap : Bp) + kbyte;
-        const uint32_t to = lds_base + slot + i * 4096, off = voff[H][i];
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base)
-                     : "m0");
+        const uint32_t to = lds_base + slot + i * 4096;
+        const Off off = voff[H][i];
+        if constexpr (WIDE)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(base + off) : "m0");
+        else
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base)
+                         : "m0");
     };
     const uint32_t nsteps = (ke - kb) / 32, last_k = (nsteps / 2 - 1) * 128;
     auto kat = [&](uint32_t half) { return min(half / 2 * 128, last_k); }; // halves past the end repeat the last K
@@ -804,19 +809,19 @@ static hipError_t launch_tile(hipStream_t st, const uint16_t *A, const uint16_t 
     return hipGetLastError();
 }
 
-template <int BM, int BN, int EPI, bool SPLIT>
+template <int BM, int BN, int EPI, bool SPLIT, bool WIDE = false>
 static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                 uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
                                 uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
 {
     static uint64_t attr_devs = 0; // devices on which the LDS limit is raised for this kernel
     const size_t lds = (size_t)gemm_ring<BM, BN>() * (BM + BN) * 64;
-    hipError_t e = lds_attr_once((const void *)gemm32_kernel<BM, BN, EPI, SPLIT>, lds, attr_devs);
+    hipError_t e = lds_attr_once((const void *)gemm32_kernel<BM, BN, EPI, SPLIT, WIDE>, lds, attr_devs);
     if (e != hipSuccess)
         return e;
     const uint32_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, total = tm * tn;
     const uint32_t grid = (total + 7) / 8 * 8;
-    gemm32_kernel<BM, BN, EPI, SPLIT><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
+    gemm32_kernel<BM, BN, EPI, SPLIT, WIDE><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
         A, B.p, B.p2, C, work, M, N, K, ldc, split, kchunk, tm, total, n_base, rope ? *rope : GemmRope{});
     return hipGetLastError();
 }
@@ -935,9 +940,12 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
     if ((uint64_t)N * K >= (1ull << 32)) // B row offsets are 32-bit
         return hipErrorInvalidValue;
     if constexpr (is_dual(EPI))
-        if (K % kBK != 0 || K > kGemm32MaxK || N % 64 != 0 || N != (2 * split + 63) / 64 * 64 || split % 8 != 0 || !B.p2 || ldc % 8 != 0 ||
-            (uintptr_t)C % 16 != 0)
+        if (K % kBK != 0 || (EPI == GEMM_FFN && K > kGemm32MaxK) || N % 64 != 0 || N != (2 * split + 63) / 64 * 64 ||
+            split % 8 != 0 || !B.p2 || ldc % 8 != 0 || (uintptr_t)C % 16 != 0)
             return hipErrorInvalidValue;
+    if constexpr (EPI == GEMM_SWIGLU)
+        if (K > kGemm32MaxK) // (fewer than 1024 rows of B: one small tile shape)
+            return launch_tile32<64, 128, EPI, false, true>(st, A, B, C, nullptr, M, N, K, ldc, split, 1, K);
     // (gemm32_kernel's copies address a tile's rows by 32-bit byte offsets; longer rows take gemm_kernel)
     if (K % kBK == 0 && K <= kGemm32MaxK)
     {

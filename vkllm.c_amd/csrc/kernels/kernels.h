@@ -288,7 +288,8 @@ struct GemmNorm
     float eps;
     bool xt = false;
 };
-// longest rows of the K % 64 == 0 tile kernel (320 of them span less than 4 GB); the dual and QKV epilogues need it
+// longest rows that the K % 64 == 0 tile kernel addresses by 32-bit offsets (320 of them span less than 4 GB); the FFN
+// operator's and the QKV epilogue need it
 constexpr uint32_t kGemm32MaxK = 1u << 22;
 // C[M, N] (row stride ldc) = A[M, K] . B[N, K]^T, fp16 operands, fp32 accumulation on MFMA. K % 8 == 0.
 // `work` (work_elems floats) holds split-K partial tiles for short prompts; with too little of it K is not split.
