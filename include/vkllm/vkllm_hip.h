@@ -121,6 +121,13 @@ extern vkllm_err_t vkllm_hip_gemm(struct vkllm_context *context, int epi, const 
                                   uint16_t *C, uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split,
                                   float *work, uint64_t work_elems);
 
+/* The tile and the K ranges that vkllm_hip_gemm and the fused step's tile GEMM run an M x N x K product on, on a GPU of
+ * `cus` compute units with `work_elems` floats for partial tiles (N counts the rows of B, both matrices' for the SwiGLU);
+ * `norm`: the residual product with the RMSNorm behind it, as the fused step runs it. A tile of 0 x 0: the fallback
+ * kernels (K % 64 != 0). Host arithmetic only: it needs no context and no GPU. */
+extern vkllm_err_t vkllm_hip_gemm_plan(uint32_t M, uint32_t N, uint32_t K, uint64_t work_elems, int norm, uint32_t cus,
+                                       uint32_t *tile_m, uint32_t *tile_n, uint32_t *splits);
+
 /* The short-prompt product of the fused step (prompts of at most 128 tokens), with vkllm_hip_gemm's arguments and
  * epilogues 0 (C = fp16(acc), ldc >= N), 2 (C = fp16(C + fp16(acc)), ldc == N, N % 32 == 0) and 3 (the SwiGLU of
  * B = [Wu; Wg], N = 2F, F % 16 == 0, ldc >= F); M <= 128, K % 16 == 0, A and B 16-byte aligned, C 8-byte aligned,

@@ -1,8 +1,8 @@
 """Parity at the kernel shapes the long workloads run, at their real widths, against the oracle.
 
 * LLaMA-2-13B widths (dim 5120, 40 heads of 128, FFN 13824), one layer, vocabulary 1000: the 2048-token prompt step
-  of the 13B workload, every row, then teacher-forced decode. That step runs the 128 x 320 residual tiles of the Wo and
-  down products, the [Wu;Wg] product in full 256 x 256 rounds plus its split-K tail, and 40-head causal attention over
+  of the 13B workload, every row, then teacher-forced decode. That step runs 128 x 320 tiles for the Wo and down
+  products, 256 x 256 for the QKV product, 256 x 192 for the [Wu;Wg] product, and 40-head causal attention over
   2048 positions.
 * LLaMA-2-7B widths (dim 4096, 32 heads of 128, FFN 11008), one layer, vocabulary 1000, a 4096-position cache: a
   4000-token prompt in four chunks, then teacher-forced decode through position 4095 on the one-launch long-cache

@@ -19,20 +19,25 @@ CASES = [
     ((1, 1, 1), 5120, 13825),   # 13B widths, odd F
     ((1, 1, 1), 11272, 40),     # longer than a wave holds: generic
     ((1, 1, 2), 64, 8),         # smallest tile product
-    ((1, 1, 37), 4096, 11008),  # whole K per 128 x 128 tile
-    ((1, 1, 129), 512, 1000),   # split K, F % 32 != 0 through the reduce
+    ((1, 1, 37), 4096, 11008),  # 7B, one row of tiles
+    ((1, 1, 129), 512, 1000),   # F % 32 != 0, whole K
+    ((1, 1, 129), 4096, 1000),  # F % 32 != 0, K split: the reduce leaves out the columns past F
+    ((1, 1, 200), 4096, 11008), # 7B, K split
     ((1, 1, 300), 320, 5000),   # F % 32 != 0 through the tile epilogue
     ((2, 3, 50), 256, 96),      # batched rows as one matrix
     ((1, 1, 1024), 256, 22016), # 256 x 256 tiles
     ((1, 1, 16), 288, 768),     # K % 64 != 0
     ((1, 1, 17), 64, 100),      # F % 8 != 0: generic
 ]
+SPLIT = {((1, 1, 129), 4096, 1000): (64, 128, 5), ((1, 1, 200), 4096, 11008): (256, 192, 2)}  # tile and K ranges
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"{'x'.join(map(str, c[0]))}-{c[1]}-{c[2]}")
 def test_ffn_up_and_gate_paths(ctx, vk, case):
     rows, K, F = case
     print(f"[ffn] rows={rows} K={K} F={F}", flush=True)
+    if case in SPLIT:
+        assert vk.gemm_plan(rows[2], (2 * F + 63) // 64 * 64, K) == SPLIT[case]
     rng = np.random.default_rng(K + F + rows[2])
     x = rng.standard_normal((*rows, K), dtype=np.float32).astype(np.float16)
     wu, wg = ((rng.standard_normal((1, 1, F, K), dtype=np.float32) / np.sqrt(K)).astype(np.float16) for _ in range(2))

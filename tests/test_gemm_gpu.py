@@ -4,10 +4,9 @@ same fp16 operands.
 The fused prompt step runs every matmul node of the reference graph (src/core/vkllm_op_matmul.c, shader
 src/shaders/vkllm_matmul.comp) through this GEMM: C = A . B^T with fp16 operands and fp32 accumulation, rounded
 once to fp16, with the SiLU or residual epilogue fused. The model tests reach it only at the tiny workload's
-sizes; these cases reach the paths that 7B and 13B prompts take: 256 x 256 tiles, the split-K tail of a partial
-last round of those tiles, one round of them with K split (residual products of long rows), 128 x 128 tiles with
-and without split K, the 64-wide fallback tiles (K not a multiple of 64), ragged M and N, and the SwiGLU epilogue
-that reads [Wu; Wg] as interleaved row blocks. The bar is the fp16 rounding of an fp32 sum:
+sizes. CASES are the products of 7B and 13B prompts and ragged ones around them; PLANNED reaches every tile of the
+kernel with whole K and with K split over workgroups, for products of one matrix and for the SwiGLU, and asserts the
+choice (vkllm_hip_gemm_plan), so that another rule cannot leave a kernel untested. The bar is the fp16 rounding of an fp32 sum:
 |C - ref| <= 1e-3 + 2e-3 |ref|, twice that for the residual and SwiGLU epilogues, which round twice.
 """
 import ctypes
@@ -20,47 +19,46 @@ pytestmark = pytest.mark.gpu
 PLAIN, SILU_HI, RESID, SWIGLU = 0, 1, 2, 3
 WORK_ELEMS = 16 << 20  # the fused step's split-K buffer (floats)
 
-# (M, N, K, epi, split, with_work): sizes assume the 256 CUs of an MI355X where a path depends on the CU count
+# (M, N, K, epi, split, with_work)
 CASES = [
-    (1024, 12288, 4096, PLAIN, 0, True),      # 7B QKV, 1024 tokens: one round of 256 x 256 tiles
-    (1024, 22016, 4096, SILU_HI, 11008, True),  # 7B gate+up: full round + split-K tail, SiLU split before the tail
-    (1024, 22016, 1024, SILU_HI, 20000, True),  # SiLU split inside the tail columns
-    (2048, 27648, 512, SILU_HI, 13824, True),   # 13B gate+up shape, 2048 tokens: three full rounds + tail
-    (1200, 15300, 1024, RESID, 0, True),      # ragged M and N through the tail split, residual epilogue
-    (2048, 5120, 512, RESID, 0, True),        # 13B Wo shape: 256 tiles of 128 x 320 instead of 160 of 256 x 256
-    (2000, 5000, 512, RESID, 0, True),        # the same rule, ragged M and N (partial 128 x 320 tiles)
-    (2048, 5120, 512, PLAIN, 0, True),        # plain epilogue: 160 tiles of 256 x 256 beat 2.5 rounds of 128 x 128
-    (1100, 9000, 256, PLAIN, 0, True),        # the same rule, ragged M and N
-    (128, 12288, 4096, PLAIN, 0, True),       # 128-token prompt: 128 x 128 tiles, split K, two K steps in flight
-    (128, 12288, 4096, PLAIN, 0, False),      # the same without a work buffer: no split
-    # prompts of <= 128 tokens with tiles for most CUs: whole K per tile, four K steps of loads in flight
+    (1024, 12288, 4096, PLAIN, 0, True),      # 7B QKV, 1024 tokens
+    (1024, 22016, 4096, SILU_HI, 11008, True),# 7B gate+up
+    (1024, 22016, 1024, SILU_HI, 20000, True),# SiLU split inside a tile
+    (2048, 27648, 512, SILU_HI, 13824, True), # 13B gate+up shape, 2048 tokens
+    (1200, 15300, 1024, RESID, 0, True),      # ragged M and N, residual epilogue
+    (2048, 5120, 512, RESID, 0, True),        # 13B Wo shape
+    (2000, 5000, 512, RESID, 0, True),        # the same, ragged M and N
+    (2048, 5120, 512, PLAIN, 0, True),        # plain epilogue
+    (1100, 9000, 256, PLAIN, 0, True),        # ragged M and N
+    (128, 12288, 4096, PLAIN, 0, True),       # 128-token prompt
+    (128, 12288, 4096, PLAIN, 0, False),      # the same without a work buffer
     (128, 22016, 4096, SILU_HI, 11008, True),  # 7B gate+up, 128 tokens
-    (128, 22016, 1216, SILU_HI, 11008, True),  # 19 K steps: four groups of four and a tail of three
+    (128, 22016, 1216, SILU_HI, 11008, True), # 19 K steps
     (100, 32000, 512, PLAIN, 0, True),        # logits shape, ragged M
     (64, 24576, 1024, RESID, 0, True),        # residual epilogue
-    (96, 24576, 128, PLAIN, 0, True),         # two K steps: tail only
-    (96, 24576, 192, PLAIN, 0, True),         # three K steps: tail only
-    (512, 4096, 4096, RESID, 0, True),        # 128 x 128 split K with the residual epilogue
-    (2048, 4096, 1024, RESID, 0, True),       # 128 x 128 tiles, enough of them that K is not split
-    # SwiGLU epilogue: B = [Wu; Wg] read as interleaved 32-row blocks, C = fp16(fp16(up) * fp16(silu(gate)))
-    (1024, 22016, 4096, SWIGLU, 11008, True),  # 7B, 1024 tokens: 256 x 256 tiles and the split-K tail
+    (96, 24576, 128, PLAIN, 0, True),         # two K steps
+    (96, 24576, 192, PLAIN, 0, True),         # three K steps
+    (512, 4096, 4096, RESID, 0, True),        # 7B Wo, 512 tokens
+    (2048, 4096, 1024, RESID, 0, True),       # 2048 tokens
+    # SwiGLU epilogue: B = [Wu; Wg] read as interleaved 16-row blocks, C = fp16(fp16(up) * fp16(silu(gate)))
+    (1024, 22016, 4096, SWIGLU, 11008, True), # 7B, 1024 tokens
     (2048, 27648, 512, SWIGLU, 13824, True),  # 13B FFN widths, 2048 tokens
-    (128, 22016, 1216, SWIGLU, 11008, True),  # 128 tokens: whole K per 128 x 128 tile, four steps in flight
-    (128, 12288, 1024, SWIGLU, 6144, True),   # 128 x 128 tiles with split K and the reduce
+    (128, 22016, 1216, SWIGLU, 11008, True),  # 128 tokens, 19 K steps
+    (128, 12288, 1024, SWIGLU, 6144, True),   # 128 tokens
     (100, 3072, 512, SWIGLU, 1536, False),    # ragged M, no work buffer
     # the LLaMA-2-13B prompt products at 2048 tokens with their real K (dim 5120, FFN 13824)
     (2048, 15360, 5120, PLAIN, 0, True),      # [Wq; Wk; Wv]
-    (2048, 5120, 5120, RESID, 0, True),       # Wo + residual: 256 tiles of 128 x 320
-    (2048, 27648, 5120, SWIGLU, 13824, True),  # [Wu; Wg] with SwiGLU: three full rounds and the split-K tail
-    (2048, 5120, 13824, RESID, 0, True),      # Wd + residual: 256 tiles of 128 x 320
+    (2048, 5120, 5120, RESID, 0, True),       # Wo + residual
+    (2048, 27648, 5120, SWIGLU, 13824, True), # [Wu; Wg] with SwiGLU
+    (2048, 5120, 13824, RESID, 0, True),      # Wd + residual
     (2048, 32000, 5120, PLAIN, 0, True),      # logits
-    # residual products with long rows whose 256 x 256 tiles leave CUs idle: K split over one round of them
-    (1024, 4096, 11008, RESID, 0, True),      # 7B Wd, 1024 tokens: 64 tiles x 4 K ranges
-    (1024, 5120, 5120, RESID, 0, True),       # 13B Wo, 1024 tokens: 80 tiles x 3
-    (640, 4096, 11008, RESID, 0, True),       # ragged last row tile: 48 tiles x 5
-    (1024, 4096, 4096, RESID, 0, True),       # 7B Wo (K 4096) stays on 128 x 128 tiles
+    # residual products with long rows
+    (1024, 4096, 11008, RESID, 0, True),      # 7B Wd, 1024 tokens
+    (1024, 5120, 5120, RESID, 0, True),       # 13B Wo, 1024 tokens
+    (640, 4096, 11008, RESID, 0, True),       # 7B Wd, 640 tokens
+    (1024, 4096, 4096, RESID, 0, True),       # 7B Wo, 1024 tokens
     (77, 1000, 256, PLAIN, 0, True),          # ragged, one partial tile row
-    (77, 1000, 1000, PLAIN, 0, True),         # K % 64 != 0: 128 x 64 tiles
+    (77, 1000, 1000, PLAIN, 0, True),         # K % 64 != 0: fallback tiles
     (300, 1000, 1000, SILU_HI, 500, True),    # K % 64 != 0, M > 128
 ]
 
@@ -125,15 +123,48 @@ def test_gemm_paths(ctx, vk, case):
                            f"{got.flat[np.argmax(err - tol)]} ref {ref.flat[np.argmax(err - tol)]}")
 
 
+# (M, N, K, epi, split, the plan: tile rows, tile columns, K ranges), on the 256 CUs of an MI355X
+PLANNED = [(M, N, K, epi, split, plan) for M, N, K, plan, epis in [
+    # K split: the partial tiles are one kernel for products of one matrix and one for SwiGLU products
+    (37, 1024, 1024, (64, 128, 4), [(SILU_HI, 500), (SWIGLU, 512)]),
+    (77, 6144, 2048, (128, 128, 5), [(RESID, 0), (SWIGLU, 3072)]),
+    (37, 12288, 2048, (128, 320, 6), [(PLAIN, 0), (SWIGLU, 6144)]),
+    (129, 4096, 5120, (192, 128, 8), [(RESID, 0), (SWIGLU, 2048)]),
+    (385, 3072, 5120, (256, 128, 5), [(SILU_HI, 1000), (SWIGLU, 1536)]),
+    (129, 12288, 5120, (256, 192, 4), [(RESID, 0), (SWIGLU, 6144)]),
+    (200, 22016, 4096, (256, 192, 2), [(SWIGLU, 11008)]),  # 7B gate/up
+    (385, 9024, 8192, (256, 256, 3), [(PLAIN, 0), (SWIGLU, 4512)]),
+    (300, 6144, 8192, (320, 128, 5), [(RESID, 0), (SWIGLU, 3072)]),
+    (129, 1000, 4096, (64, 128, 8), [(PLAIN, 0), (RESID, 0)]),
+    # whole K: a kernel an epilogue
+    (129, 1024, 1024, (64, 128, 1), [(SILU_HI, 300), (RESID, 0), (SWIGLU, 512)]),
+    (129, 12288, 1024, (128, 128, 1), [(SILU_HI, 5000), (RESID, 0), (SWIGLU, 6144)]),
+    (641, 12288, 1024, (128, 320, 1), [(SILU_HI, 5000), (RESID, 0), (SWIGLU, 6144)]),
+    (129, 22016, 1024, (192, 128, 1), [(SILU_HI, 11008), (RESID, 0), (SWIGLU, 11008)]),
+    (193, 22016, 1024, (256, 128, 1), [(SILU_HI, 11008), (RESID, 0), (SWIGLU, 11008)]),
+    (385, 22016, 1024, (256, 192, 1), [(SILU_HI, 11008), (RESID, 0), (SWIGLU, 11008)]),
+    (641, 16384, 1024, (256, 256, 1), [(SILU_HI, 9000), (RESID, 0), (SWIGLU, 8192)]),
+    (300, 22016, 1024, (320, 128, 1), [(SILU_HI, 11008), (RESID, 0), (SWIGLU, 11008)]),
+] for epi, split in epis]
+
+
+@pytest.mark.parametrize("case", PLANNED, ids=lambda c: f"{c[0]}x{c[1]}x{c[2]}-e{c[3]}-{c[5][0]}x{c[5][1]}-{c[5][2]}")
+def test_gemm_plans(ctx, vk, case):
+    M, N, K, epi, split, plan = case
+    assert vk.gemm_plan(M, N, K, WORK_ELEMS) == plan
+    test_gemm_paths(ctx, vk, (M, N, K, epi, split, True))
+
+
 def test_gemm_split_k_is_deterministic(ctx, vk):
     """The split-K reduce adds the partial tiles in a fixed order: repeated calls give identical bits."""
-    M, N, K = 1024, 22016, 1024
+    M, N, K = 129, 12288, 5120
+    assert vk.gemm_plan(M, N, K, WORK_ELEMS)[2] == 4
     rng = np.random.default_rng(5)
     a = rng.standard_normal((M, K), dtype=np.float32).astype(np.float16)
     b = (rng.standard_normal((N, K), dtype=np.float32) * (1.0 / np.sqrt(K))).astype(np.float16)
     c0 = np.zeros((M, N), np.float16)
-    first = run_gemm(ctx, vk, a, b, c0, SILU_HI, 11008, True)
-    second = run_gemm(ctx, vk, a, b, c0, SILU_HI, 11008, True)
+    first = run_gemm(ctx, vk, a, b, c0, SILU_HI, 6144, True)
+    second = run_gemm(ctx, vk, a, b, c0, SILU_HI, 6144, True)
     assert np.array_equal(first.view(np.uint16), second.view(np.uint16))
 
 

@@ -117,7 +117,7 @@ def test_streamed_prefill_matches_oracle(ctx, vk, oracle, prompt_len):
 
 
 def test_streamed_prefill_against_tile_gemms(ctx, vk, monkeypatch):
-    """The same 100-token prompt step with and without the tiled copies (VKLLM_PREFILL_TILED=0: the 128 x 128 tile
+    """The same 100-token prompt step with and without the tiled copies (VKLLM_PREFILL_TILED=0: the tile
     GEMMs): identical greedy ids; logits within 2e-2 (the two sum in different orders)."""
     from test_model_gpu import LOGIT_TOL, _device_loop
 

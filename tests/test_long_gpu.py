@@ -98,7 +98,7 @@ def test_prompt_2048_tokens(ctx, vk, oracle, chunks):
 
 def test_long_cache_decode_at_7b_widths(ctx, vk, oracle):
     """The 7B widths (dim 4096, 32 heads of 128, FFN 11008; one layer, vocabulary 1000): a 1030-token prompt (256 x 256
-    tiles with a ragged last row block, the down product split over K), then decode past the 1024-position
+    tiles with a ragged last row block, the output and down products split over K), then decode past the 1024-position
     switch-over on the one-launch long-cache attention (32 heads x 5 chunks, every chunk block resident) with the
     oracle's ids fed back."""
     shape = dict(n_layer=1, dim=4096, n_head=32, ffn=11008, vocab=1000, ctx=1100)

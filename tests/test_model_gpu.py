@@ -179,7 +179,7 @@ def test_7b_widths_two_layers(ctx, vk, oracle):
 @pytest.mark.parametrize("dim,heads,ffn", [(4096, 32, 11008), (5120, 40, 13824)], ids=["7b", "13b"])
 def test_300_token_prompt_at_real_widths(ctx, vk, oracle, dim, heads, ffn):
     """A 300-token prompt at the 7B and 13B widths (one layer, vocabulary 1000 to keep the oracle quick): the down
-    product (K 11008 / 13824) splits K 8 / 6 ways over one round of 256 x 256 tiles, and the reduce adds the residual
+    product (K 11008 / 13824) splits K 4 / 6 ways over 192 x 128 / 320 x 128 tiles, and the reduce adds the residual
     and the next RMSNorm. Every prompt row against the oracle (logits within 2e-2, ids identical but at one-ulp
     ties), then 3 decode steps fed the oracle's ids (free-running streams part at the first one-ulp tie: with seed 13
     the 13B widths have one at the first decode step, top-2 logits 0.0039 apart)."""
@@ -283,13 +283,19 @@ def test_arg_max_in_the_vocabulary_product(ctx, vk, monkeypatch):
         assert int(ids_a[step]) == argmax_tie_rule(row) and int(ids_a[step]) in (70, 20000)
 
 
-@pytest.mark.parametrize("prompt_len", [100, 300, 1030])
-def test_qkv_rope_epilogue_matches_separate_kernel(ctx, vk, monkeypatch, prompt_len):
+@pytest.mark.parametrize("prompt_len,dim,plan", [
+    (100, 4096, (64, 128, 1)), (300, 4096, (192, 128, 1)), (400, 4096, (256, 192, 2)), (1030, 4096, (256, 256, 1)),
+    (20, 768, (64, 128, 3)), (100, 1920, (128, 128, 5)), (2048, 576, (128, 128, 1)), (2048, 704, (192, 128, 1)),
+    (2048, 1024, (256, 128, 1)), (2048, 1408, (320, 128, 1)), (2048, 1600, (128, 320, 1)), (2048, 1728, (256, 192, 1))])
+def test_qkv_rope_epilogue_matches_separate_kernel(ctx, vk, monkeypatch, prompt_len, dim, plan):
     """RoPE and the K/V append in the prompt step's QKV product epilogue against the stored product and the separate
-    RoPE kernel (src/shaders/vkllm_rope.comp, src/shaders/vkllm_update_rows.comp), at the 7B widths: the split-K reduce
-    (100 tokens), 128 x 128 tiles (300) and 256 x 256 tiles with a ragged last row block (1030), then decode steps
-    reading the appended cache; identical ids and logits."""
-    shape = dict(n_layer=2, dim=4096, n_head=32, ffn=11008, vocab=32000, ctx=1100)
+    RoPE kernel (src/shaders/vkllm_rope.comp, src/shaders/vkllm_update_rows.comp), at the 7B widths and, for the other
+    tiles, at narrow ones with heads of 64: every tile, and K split with the reduce behind it (`plan`: tile and K
+    ranges), then decode steps reading the appended cache; identical ids and logits."""
+    wide = dim == 4096
+    shape = dict(n_layer=2, dim=dim, n_head=32 if wide else dim // 64, ffn=11008 if wide else 512,
+                 vocab=32000 if wide else 1000, ctx=prompt_len + 70)
+    assert vk.gemm_plan(prompt_len, 3 * dim, dim) == plan
     prompt = vk.prompt_tokens(9, prompt_len, shape["vocab"])
     # both arms on the tile GEMMs (the streamed short-prompt products need the epilogue and sum in another order)
     monkeypatch.setenv("VKLLM_PREFILL_TILED", "0")

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 CASES = [
     (288, 6, 768, 1000, 64, 16, 17),
     (288, 6, 768, 1000, 64, 2, 1),
-    (288, 6, 768, 32000, 64, 15, 3),
+    (288, 6, 768, 32000, 64, 15, 3),   # 2000 tiles of logits, on the small kernel
+    (288, 6, 768, 32000, 64, 33, 3),   # 6000: the tile GEMM
     (288, 6, 768, 1001, 48, 33, 15),   # kv == head size at the end
     (96, 4, 1024, 500, 320, 256, 2),
     (96, 4, 1024, 500, 320, 257, 2),   # past the longest small step

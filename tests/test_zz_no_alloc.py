@@ -47,16 +47,21 @@ def _run(ctx, vk, a, b, c0, epi, split, work_elems, noalloc):
                 ctx.free(t)
 
 
-# (M, N, K, epi, split, work_elems): each pair is run back to back, the second product smaller than the first
+# (M, N, K, epi, split, work_elems): each pair is run back to back, the second product smaller than the first. The last
+# two pairs split K in both products (asserted), so the second's partial tiles lie over the first's.
 PAIRS = [
     ((128, 12288, 4096, PLAIN, 0, MAX_WORK), (64, 4096, 1024, RESID, 0, 1 << 20)),
     ((128, 22016, 1024, SWIGLU, 11008, MAX_WORK), (100, 3072, 512, SILU_HI, 1536, 2 << 20)),
     ((512, 4096, 4096, RESID, 0, MAX_WORK), (77, 1000, 1000, PLAIN, 0, MAX_WORK)),
+    ((385, 3072, 5120, PLAIN, 0, MAX_WORK), (77, 1000, 4096, SILU_HI, 500, MAX_WORK)),
+    ((129, 4096, 5120, SWIGLU, 2048, MAX_WORK), (37, 1024, 1024, SWIGLU, 512, 1 << 18)),
 ]
 
 
 @pytest.mark.parametrize("pair", PAIRS, ids=lambda p: f"{p[0][0]}x{p[0][1]}x{p[0][2]}-then-{p[1][0]}x{p[1][1]}x{p[1][2]}")
 def test_noalloc_gemm_matches_gemm_with_work_buffer(ctx, vk, pair):
+    if pair in PAIRS[-2:]:
+        assert all(vk.gemm_plan(M, N, K, work)[2] > 1 for M, N, K, _, _, work in pair)
     rng = np.random.default_rng(sum(pair[0][:3]) + pair[1][0])
     ops = [_operands(rng, M, N, K, epi, split) for (M, N, K, epi, split, _) in pair]
     got = []
@@ -97,7 +102,8 @@ def test_noalloc_gemm_under_stream_capture(ctx, vk):
     """One split-K call captured into a hipGraph (global capture mode, where an allocating call would fail the
     capture), replayed three times with eager calls of other shapes between the replays (each overwrites the shared
     scratch): every replay's output is bit-identical to the eager call's."""
-    M, N, K = 64, 1024, 8192  # 8 tiles of 128 x 128 on 256 CUs: K is split, the partials go through the scratch
+    M, N, K = 64, 1024, 8192
+    assert vk.gemm_plan(M, N, K, MAX_WORK)[2] > 1  # the partials go through the scratch
     rng = np.random.default_rng(5)
     a, b, c0 = _operands(rng, M, N, K, PLAIN, 0)
     want = _run(ctx, vk, a, b, c0, PLAIN, 0, MAX_WORK, noalloc=True)
@@ -116,14 +122,15 @@ def test_noalloc_gemm_under_stream_capture(ctx, vk):
         end = H.hipStreamEndCapture(stream, ctypes.byref(graph))
         assert rc == vk.ERR_OK and end == 0, (rc, end)
         assert H.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
-        other = _operands(rng, 100, 3072, 512, SILU_HI, 1536)
+        other = _operands(rng, 77, 1000, 4096, SILU_HI, 500)
+        assert vk.gemm_plan(77, 1000, 4096, MAX_WORK)[2] > 1
         for rep in range(3):
             ctx.upload(tc, np.zeros((M, N), np.float16))
             assert H.hipGraphLaunch(exe, stream) == 0
             assert H.hipStreamSynchronize(stream) == 0
             got = ctx.download(tc).reshape(M, N)
             assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), f"replay {rep} differs"
-            _run(ctx, vk, *other, SILU_HI, 1536, 2 << 20, noalloc=True)  # eager work on the same scratch
+            _run(ctx, vk, *other, SILU_HI, 500, MAX_WORK, noalloc=True)  # eager work on the same scratch
     finally:
         if exe.value:
             H.hipGraphExecDestroy(exe)

@@ -1454,6 +1454,17 @@ extern "C" vkllm_err_t vkllm_hip_gemm_streamed(struct vkllm_context *ctx, int ep
     return VKLLM_ERR_OK;
 }
 
+extern "C" vkllm_err_t vkllm_hip_gemm_plan(uint32_t M, uint32_t N, uint32_t K, uint64_t work_elems, int norm,
+                                           uint32_t cus, uint32_t *tile_m, uint32_t *tile_n, uint32_t *splits)
+{
+    _CHECK_ARGS(M > 0 && N > 0 && K >= 8 && K % 8 == 0 && cus > 0 && tile_m && tile_n && splits);
+    const vk::GemmPlan p = vk::gemm_plan(M, N, K, cus, (size_t)work_elems, norm != 0);
+    *tile_m = p.tile_m;
+    *tile_n = p.tile_n;
+    *splits = p.splits;
+    return VKLLM_ERR_OK;
+}
+
 extern "C" vkllm_err_t vkllm_hip_gemm(struct vkllm_context *ctx, int epi, const uint16_t *A, const uint16_t *B,
                                       uint16_t *C, uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split,
                                       float *work, uint64_t work_elems)

@@ -878,7 +878,7 @@ static hipError_t launch_choice(hipStream_t st, int tile, const uint16_t *A, Gem
 struct TileChoice
 {
     int tile;
-    uint32_t splits;
+    uint32_t splits, kchunk; // K ranges of kchunk
 };
 
 // Time of a product on one tile shape with K in `splits` ranges, us: the tile's measured step, or what the busy CUs
@@ -908,7 +908,7 @@ static float tile_time(uint32_t M, uint32_t N, uint32_t K, TileShape t, uint32_t
 
 static TileChoice pick_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, size_t work_elems, bool norm)
 {
-    TileChoice best{0, 1};
+    TileChoice best{0, 1, K};
     float best_us = FLT_MAX;
     for (int i = 0; i < kTileCount; ++i)
         for (uint32_t s = 1; s <= 8; ++s) // (more were at most 2% faster anywhere, with more partials to round)
@@ -920,10 +920,23 @@ static TileChoice pick_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, si
             if (us < best_us)
             {
                 best_us = us;
-                best = {i, s};
+                best = {i, s, K};
             }
         }
+    if (best.splits > 1)
+    {
+        best.kchunk = ((K + best.splits - 1) / best.splits + kBK - 1) / kBK * kBK;
+        best.splits = (K + best.kchunk - 1) / best.kchunk;
+    }
     return best;
+}
+
+GemmPlan gemm_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, size_t work_elems, bool norm)
+{
+    if (K % kBK != 0 || K > kGemm32MaxK)
+        return {0, 0, 0};
+    const TileChoice c = pick_tile(M, N, K, cus, work_elems, norm);
+    return {kTiles[c.tile].bm, kTiles[c.tile].bn, c.splits};
 }
 
 template <int EPI>
@@ -950,7 +963,7 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
     if (K % kBK == 0 && K <= kGemm32MaxK)
     {
         const TileChoice c = pick_tile(M, N, K, cus, work_elems, EPI == GEMM_RESID && norm);
-        const uint32_t kchunk = ((K + c.splits - 1) / c.splits + kBK - 1) / kBK * kBK, splits = (K + kchunk - 1) / kchunk;
+        const uint32_t kchunk = c.kchunk, splits = c.splits;
         if (splits <= 1)
             return launch_choice<EPI, false>(st, c.tile, A, B, C, nullptr, M, N, K, ldc, split, 1, K, rope);
         // the partial tiles are the same for every epilogue: one kernel for products of one matrix, one for dual ones

@@ -299,6 +299,13 @@ hipError_t launch_gemm(hipStream_t st, int epi, const uint16_t *A, const uint16_
                        uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, int cu_count, float *work,
                        size_t work_elems, const GemmRope *rope = nullptr, const GemmNorm *norm = nullptr,
                        const uint16_t *B2 = nullptr);
+// the tile and K ranges that launch_gemm runs such a product on, by the same rule (N: the dual products' columns of both
+// matrices; norm: GEMM_RESID's); {0, 0, 0} where it takes the fallback tiles
+struct GemmPlan
+{
+    uint32_t tile_m, tile_n, splits;
+};
+GemmPlan gemm_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, size_t work_elems, bool norm);
 // The same for small models, one launch with the RMSNorm of A's rows in front (norm_w): GEMM_PLAIN, GEMM_SWIGLU (B up
 // rows, B2 gate rows, N = F) and GEMM_QKV_ROPE with it, GEMM_RESID and GEMM_FFN without. C is [M, N] packed, rows
 // 16-byte aligned in A and B, N even, K % 32 == 0 and at most kGemmSmallMaxK; the head size even.

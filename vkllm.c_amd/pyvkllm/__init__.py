@@ -220,6 +220,7 @@ def lib():
             "vkllm_hip_model_last_logits": (E, [vp, ctypes.POINTER(ModelStruct), vp, u32]),
             "vkllm_hip_token_loop": (E, [vp, ctypes.POINTER(ModelStruct), vp, u32, u32, u32, vp, vp, vp]),
             "vkllm_hip_gemm": (E, [vp, E, vp, vp, vp, u32, u32, u32, u32, u32, vp, ctypes.c_uint64]),
+            "vkllm_hip_gemm_plan": (E, [u32, u32, u32, ctypes.c_uint64, E, u32] + 3 * [ctypes.POINTER(u32)]),
             "vkllm_hip_gemm_noalloc": (E, [vp, E, vp, vp, vp, u32, u32, u32, u32, u32, ctypes.c_uint64]),
             "vkllm_hip_gemm_streamed": (E, [vp, E, vp, vp, vp, u32, u32, u32, u32, u32]),
             "vkllm_hip_abi_layout": (E, [ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(ctypes.c_uint64), E]),
@@ -294,6 +295,13 @@ def abi_check():
 
 
 # --------------------------------------------------------------------------------------------------------------
+def gemm_plan(M, N, K, work_elems=16 << 20, norm=False, cus=256):
+    """(tile rows, tile columns, K ranges) of the tile GEMM for a product (vkllm_hip_gemm_plan)."""
+    out = [ctypes.c_uint32() for _ in range(3)]
+    check("vkllm_hip_gemm_plan", lib().vkllm_hip_gemm_plan(M, N, K, work_elems, norm, cus, *map(ctypes.byref, out)))
+    return tuple(x.value for x in out)
+
+
 class Ctx:
     """A vkllm_context plus one commands object for op-level work."""
 
