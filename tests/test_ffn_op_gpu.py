@@ -24,6 +24,7 @@ CASES = [
     ((1, 1, 129), 4096, 1000),  # F % 32 != 0, K split: the reduce leaves out the columns past F
     ((1, 1, 200), 4096, 11008), # 7B, K split
     ((1, 1, 300), 320, 5000),   # F % 32 != 0 through the tile epilogue
+    ((1, 1, 300), 192, 5000),   # the same, rows shorter than the ring
     ((2, 3, 50), 256, 96),      # batched rows as one matrix
     ((1, 1, 1024), 256, 22016), # 256 x 256 tiles
     ((1, 1, 16), 288, 768),     # K % 64 != 0

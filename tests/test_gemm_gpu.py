@@ -145,6 +145,12 @@ PLANNED = [(M, N, K, epi, split, plan) for M, N, K, plan, epis in [
     (385, 22016, 1024, (256, 192, 1), [(SILU_HI, 11008), (RESID, 0), (SWIGLU, 11008)]),
     (641, 16384, 1024, (256, 256, 1), [(SILU_HI, 9000), (RESID, 0), (SWIGLU, 8192)]),
     (300, 22016, 1024, (320, 128, 1), [(SILU_HI, 11008), (RESID, 0), (SWIGLU, 11008)]),
+    # rows shorter than the ring (the 128 x 128 tile with two workgroups a CU): fewer halves than it is filled with, as
+    # many, and one step more; ragged M and N
+    (301, 8200, 64, (128, 128, 1), [(SILU_HI, 3000), (RESID, 0)]),
+    (301, 8256, 64, (128, 128, 1), [(SWIGLU, 4128)]),
+    (513, 9000, 128, (128, 128, 1), [(SILU_HI, 3000), (RESID, 0)]),
+    (1000, 8064, 192, (128, 128, 1), [(SILU_HI, 3000), (RESID, 0), (SWIGLU, 4032)]),
 ] for epi, split in epis]
 
 

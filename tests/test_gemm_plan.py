@@ -33,5 +33,16 @@ def test_plans_fit_the_scratch(plan):
         assert splits == 1 or K // splits >= 192  # 256 of K a range, less what the ranges' rounding to 64 moves
 
 
+@pytest.mark.parametrize("M,N", [(640, 8192), (1024, 8192), (2048, 4096), (4096, 2048), (4096, 16384)])
+def test_short_rows(plan, M, N):
+    """Products of short rows are their workgroups' starts and epilogues: up to K 192 two workgroups of 128 x 128 a CU (on
+    one large tile a CU 2048 x 4096 x 64 takes 8.3 us instead of 7.3); up to K 512 not 256 x 128, which ran at 10.7 or at
+    17 us (2048 x 4096 x 256) from one run to the next."""
+    for K in (64, 128, 192):
+        assert plan(M, N, K) == (128, 128, 1)
+    for K in (256, 320, 512):
+        assert plan(M, N, K)[:2] != (256, 128)
+
+
 def test_fallback_products_have_no_tile(plan):
     assert plan(77, 1000, 1000) == (0, 0, 0) and plan(2, 8, (1 << 22) + 64) == (0, 0, 0)

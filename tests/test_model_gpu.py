@@ -285,7 +285,7 @@ def test_arg_max_in_the_vocabulary_product(ctx, vk, monkeypatch):
 
 @pytest.mark.parametrize("prompt_len,dim,plan", [
     (100, 4096, (64, 128, 1)), (300, 4096, (192, 128, 1)), (400, 4096, (256, 192, 2)), (1030, 4096, (256, 256, 1)),
-    (20, 768, (64, 128, 3)), (100, 1920, (128, 128, 5)), (2048, 576, (128, 128, 1)), (2048, 704, (192, 128, 1)),
+    (20, 768, (64, 128, 3)), (100, 1920, (128, 128, 5)), (2048, 576, (128, 128, 1)), (4000, 192, (128, 128, 1)), (2048, 704, (192, 128, 1)),
     (2048, 1024, (256, 128, 1)), (2048, 1408, (320, 128, 1)), (2048, 1600, (128, 320, 1)), (2048, 1728, (256, 192, 1))])
 def test_qkv_rope_epilogue_matches_separate_kernel(ctx, vk, monkeypatch, prompt_len, dim, plan):
     """RoPE and the K/V append in the prompt step's QKV product epilogue against the stored product and the separate

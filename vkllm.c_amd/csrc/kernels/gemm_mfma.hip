@@ -254,17 +254,10 @@ __host__ __device__ __forceinline__ void for_seq(std::integer_sequence<int, J...
     (f(std::integral_constant<int, J>{}), ...);
 }
 
-// halves in the LDS ring: as many as fit 160 KB, up to 10
-template <int BM, int BN> constexpr int gemm_ring()
-{
-    constexpr int fit = 160 * 1024 / ((BM + BN) * 64);
-    return fit < 10 ? fit : 10;
-}
-
 // n_base: product column of the kernel's column 0 (B rows and C columns are addressed from it; N counts the
-// kernel's columns). WIDE: rows of any length, a tile's rows by 64-bit offsets (otherwise K <= kGemm32MaxK). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
+// kernel's columns). NH: halves in the LDS ring. WIDE: rows of any length, a tile's rows by 64-bit offsets (otherwise K <= kGemm32MaxK). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
 // blocks and `split` holds F.
-template <int BM, int BN, int EPI, bool SPLIT, bool WIDE = false>
+template <int BM, int BN, int NH, int EPI, bool SPLIT, bool WIDE = false>
 __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                         const uint16_t *__restrict__ B2, uint16_t *C, float *work,
                                                         uint32_t M, uint32_t N, uint32_t K, uint32_t ldc,
@@ -272,7 +265,7 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
                                                         uint32_t tiles_total, uint32_t n_base, GemmRope rope)
 {
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int HALF = (BM + BN) * 64, NH = gemm_ring<BM, BN>(); // bytes of a half, halves in the ring
+    constexpr int HALF = (BM + BN) * 64; // bytes of a half
     constexpr int ND = (BM + BN) / 64, NAI = WM / 32; // copies of a wave per half, the first NAI of them rows of A
     constexpr int NR = 2 * (TM + TN), NM = 2 * TM * TN; // operand reads and MFMAs of a step
     static_assert(WM % 32 == 0 && WN % 32 == 0 && NH >= 5, "whole MFMA blocks, and the waits below");
@@ -310,19 +303,29 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
             voff[h][i] = (Off)row * K * 2 + ((lane ^ (r & 7)) & 7) * 16;
         }
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)lds + wid * 1024;
-    auto copy = [&](auto h_tag, int i, uint32_t slot, uint32_t kbyte) {
+    const uint32_t nsteps = (ke - kb) / 32; // and halves
+    // ENDS: the half may lie past the end, and is then copied by no lane (EXEC 0; every lane is active here): it moves
+    // nothing and still counts, so the waits below stay constant. Copying the last K over and over in its place took
+    // 2048 x 16384 x 256 from 39 to 47 us; the steps whose halves all exist leave the test out (0.9% of long products).
+    auto copy = [&](auto h_tag, auto ends_tag, int i, uint32_t slot, uint32_t half) {
         constexpr int H = decltype(h_tag)::value;
-        const char *base = (i < NAI ? Ap : Bp) + kbyte;
-        const uint32_t to = lds_base + slot + i * 4096;
+        const char *base = (i < NAI ? Ap : Bp) + half / 2 * 128;
+        const uint32_t to = lds_base + slot + i * 4096, end = nsteps;
         const Off off = voff[H][i];
         if constexpr (WIDE)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(base + off) : "m0");
+            asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lt_u32 %2, %3\n\ts_cselect_b64 exec, -1, 0\n\t"
+                         "global_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(to),
+                         "v"(base + off), "s"(half), "s"(end)
+                         : "m0", "scc");
+        else if constexpr (decltype(ends_tag)::value)
+            asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lt_u32 %3, %4\n\ts_cselect_b64 exec, -1, 0\n\t"
+                         "global_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(to),
+                         "v"(off), "s"(base), "s"(half), "s"(end)
+                         : "m0", "scc");
         else
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base)
                          : "m0");
     };
-    const uint32_t nsteps = (ke - kb) / 32, last_k = (nsteps / 2 - 1) * 128;
-    auto kat = [&](uint32_t half) { return min(half / 2 * 128, last_k); }; // halves past the end repeat the last K
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
     using I1 = std::integral_constant<int, 1>;
     // One step: the MFMAs of register set S, the reads of the next step (K offset 32 P) into the other set, and this
     // wave's copies of a half with parity H into `slot`
-    auto step = [&](auto s_tag, auto p_tag, auto h_tag, uint32_t slot, uint32_t kbyte) {
+    auto step = [&](auto s_tag, auto p_tag, auto h_tag, auto ends_tag, uint32_t slot, uint32_t half) {
         constexpr int S = decltype(s_tag)::value;
         using Other = std::integral_constant<int, 1 - S>;
         int nr = 0, nd = 0;
@@ -365,7 +368,7 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (; nd < want_d; ++nd)
-                copy(h_tag, nd, slot, kbyte);
+                copy(h_tag, ends_tag, nd, slot, half);
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
             read(Other{}, nr / (TM + TN), nr % (TM + TN), decltype(p_tag)::value);
 #pragma unroll
         for (; nd < ND; ++nd)
-            copy(h_tag, nd, slot, kbyte);
+            copy(h_tag, ends_tag, nd, slot, half);
     };
     auto next_slot = [&](uint32_t o, uint32_t by) { return o + by >= NH * HALF ? o + by - NH * HALF : o + by; };
 
@@ -381,7 +384,7 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
         constexpr int J = decltype(j)::value;
 #pragma unroll
         for (int i = 0; i < ND; ++i)
-            copy(std::integral_constant<int, J % 2>{}, i, J * HALF, kat(J));
+            copy(std::integral_constant<int, J % 2>{}, std::true_type{}, i, J * HALF, J);
     });
     // halves 0 and 1 have landed in every wave
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NH - 3) * ND) : "memory");
@@ -389,9 +392,8 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
     for (int x = 0; x < NR; ++x)
         read(I0{}, x / (TM + TN), x % (TM + TN), 0);
     uint32_t slot = (NH - 1) * HALF;
-    for (uint32_t s = 0; s < nsteps; s += 2)
-    {
-        step(I0{}, I1{}, std::integral_constant<int, (NH - 1) % 2>{}, slot, kat(s + NH - 1));
+    auto pair = [&](auto ends_tag, uint32_t s) {
+        step(I0{}, I1{}, std::integral_constant<int, (NH - 1) % 2>{}, ends_tag, slot, s + NH - 1);
         slot = next_slot(slot, HALF);
         // of the halves requested so far all but the last NH - 4 have landed, halves s + 2 and s + 3 among them, and
         // every wave has read all of halves s and s + 1
@@ -399,10 +401,15 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
         __builtin_amdgcn_sched_barrier(0);
         slot_a = next_slot(slot_a, 2 * HALF);
         slot_b = next_slot(slot_b - WM * 128, 2 * HALF) + WM * 128;
-        step(I1{}, I0{}, std::integral_constant<int, NH % 2>{}, slot, kat(s + NH));
+        step(I1{}, I0{}, std::integral_constant<int, NH % 2>{}, ends_tag, slot, s + NH);
         slot = next_slot(slot, HALF);
-    }
-    // the copies past the end have landed before the ring is used again
+    };
+    uint32_t s = 0;
+    for (; s + NH < nsteps; s += 2)
+        pair(std::false_type{}, s);
+    for (; s < nsteps; s += 2)
+        pair(std::true_type{}, s);
+    // nothing is in flight when the ring is used again
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
     if constexpr (!SPLIT)
@@ -809,19 +816,19 @@ static hipError_t launch_tile(hipStream_t st, const uint16_t *A, const uint16_t 
     return hipGetLastError();
 }
 
-template <int BM, int BN, int EPI, bool SPLIT, bool WIDE = false>
+template <int BM, int BN, int NH, int EPI, bool SPLIT, bool WIDE = false>
 static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                 uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
                                 uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
 {
     static uint64_t attr_devs = 0; // devices on which the LDS limit is raised for this kernel
-    const size_t lds = (size_t)gemm_ring<BM, BN>() * (BM + BN) * 64;
-    hipError_t e = lds_attr_once((const void *)gemm32_kernel<BM, BN, EPI, SPLIT, WIDE>, lds, attr_devs);
+    const size_t lds = (size_t)NH * (BM + BN) * 64;
+    hipError_t e = lds_attr_once((const void *)gemm32_kernel<BM, BN, NH, EPI, SPLIT, WIDE>, lds, attr_devs);
     if (e != hipSuccess)
         return e;
     const uint32_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, total = tm * tn;
     const uint32_t grid = (total + 7) / 8 * 8;
-    gemm32_kernel<BM, BN, EPI, SPLIT, WIDE><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
+    gemm32_kernel<BM, BN, NH, EPI, SPLIT, WIDE><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
         A, B.p, B.p2, C, work, M, N, K, ldc, split, kchunk, tm, total, n_base, rope ? *rope : GemmRope{});
     return hipGetLastError();
 }
@@ -855,10 +862,19 @@ static hipError_t launch_shape(hipStream_t st, const uint16_t *A, const uint16_t
 struct TileShape
 {
     uint16_t bm, bn;
+    // halves in the LDS ring (as many as fit 160 KB, up to 10, but for the last tile), workgroups that fit a CU with it
+    uint8_t ring, per_cu;
     float step_us; // 64 of K on one of many busy CUs, measured (products of 64 to 216 such steps in one round)
 };
-constexpr TileShape kTiles[] = {{256, 256, 1.29f}, {256, 192, 1.18f}, {256, 128, 0.88f}, {128, 320, 1.18f},
-                                {320, 128, 1.05f}, {192, 128, 0.66f}, {128, 128, 0.50f}, {64, 128, 0.36f}};
+constexpr TileShape kTiles[] = {{256, 256, 5, 1, 1.29f}, {256, 192, 5, 1, 1.18f}, {256, 128, 6, 1, 0.88f},
+                                {128, 320, 5, 1, 1.18f}, {320, 128, 5, 1, 1.05f}, {192, 128, 8, 1, 0.66f},
+                                {128, 128, 10, 1, 0.50f}, {64, 128, 10, 1, 0.36f}, {128, 128, 5, 2, 0.50f}};
+// Products of short rows are their workgroups' starts and epilogues. With K of at most kShortK the 128 x 128 tile takes
+// a ring of 5, so that two workgroups of a CU cover each other's (longer rows wait for that ring). us, ring of 10 / 5
+// and the tile that was fastest without it: 2048 x 4096 x 64 10.0 / 7.4 (8.3 on 256 x 128), 2048 x 16384 x 192 39.3 /
+// 26.6 (30.8), 1024 x 4096 x 128 6.5 / 5.8; K 320: 13.0 / 11.3 to 14.4 from run to run. So varies 256 x 128 up to K
+// 512 (2048 x 4096 x 256 10.7 to 17.0, x 320 13.4 to 18.3), which is left out there: 320 x 128 takes 11.5 and 12.6.
+constexpr uint32_t kShortK = 192, kMidK = 512;
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
 template <int EPI, bool SPLIT>
@@ -870,7 +886,7 @@ static hipError_t launch_choice(hipStream_t st, int tile, const uint16_t *A, Gem
     for_seq(std::make_integer_sequence<int, kTileCount>{}, [&](auto i) {
         constexpr TileShape T = kTiles[decltype(i)::value];
         if (tile == decltype(i)::value)
-            e = launch_tile32<T.bm, T.bn, EPI, SPLIT>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, 0, rope);
+            e = launch_tile32<T.bm, T.bn, T.ring, EPI, SPLIT>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, 0, rope);
     });
     return e;
 }
@@ -892,8 +908,10 @@ static float tile_time(uint32_t M, uint32_t N, uint32_t K, TileShape t, uint32_t
     const uint32_t steps = (K / kBK + splits - 1) / splits;
     const float flop = 2.f * t.bm * t.bn * kBK, area = t.bm * t.bn / 65536.f;
     auto round = [&](float n) { return steps * std::max(t.step_us, n * flop / 1.3e9f) + 5.f + 5.f * area; };
-    const uint64_t full = wgs / cus, rest = wgs % cus;
-    float us = full * round((float)cus) + (rest ? round((float)rest) : 0.f);
+    const uint64_t slots = (uint64_t)cus * t.per_cu, full = wgs / slots, rest = wgs % slots;
+    float us = full * round((float)slots) + (rest ? round((float)rest) : 0.f);
+    if (t.per_cu > 1 && wgs > slots) // a round's epilogues run under the next one's start
+        us -= 2.8f * (full + (rest ? 1 : 0) - 1);
     // several rows of tiles share the weights through L2 at some cost; the last term: of tiles that all wait for the
     // weights, the one that is done soonest
     const float weights = (float)N * K * 2 * (M > t.bm ? 1.2f : 1.f);
@@ -911,18 +929,23 @@ static TileChoice pick_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, si
     TileChoice best{0, 1, K};
     float best_us = FLT_MAX;
     for (int i = 0; i < kTileCount; ++i)
+    {
+        const TileShape t = kTiles[i];
+        if (t.bn == 128 && ((t.bm == 128 && (t.per_cu > 1) != (K <= kShortK)) || (t.bm == 256 && K <= kMidK)))
+            continue;
         for (uint32_t s = 1; s <= 8; ++s) // (more were at most 2% faster anywhere, with more partials to round)
         {
             // a range keeps at least 256 of K
             if (s > 1 && (K / s < 4 * kBK || (size_t)s * M * N > work_elems))
                 break;
-            const float us = tile_time(M, N, K, kTiles[i], s, cus, norm);
+            const float us = tile_time(M, N, K, t, s, cus, norm);
             if (us < best_us)
             {
                 best_us = us;
                 best = {i, s, K};
             }
         }
+    }
     if (best.splits > 1)
     {
         best.kchunk = ((K + best.splits - 1) / best.splits + kBK - 1) / kBK * kBK;
@@ -958,7 +981,7 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
             return hipErrorInvalidValue;
     if constexpr (EPI == GEMM_SWIGLU)
         if (K > kGemm32MaxK) // (fewer than 1024 rows of B: one small tile shape)
-            return launch_tile32<64, 128, EPI, false, true>(st, A, B, C, nullptr, M, N, K, ldc, split, 1, K);
+            return launch_tile32<64, 128, 10, EPI, false, true>(st, A, B, C, nullptr, M, N, K, ldc, split, 1, K);
     // (gemm32_kernel's copies address a tile's rows by 32-bit byte offsets; longer rows take gemm_kernel)
     if (K % kBK == 0 && K <= kGemm32MaxK)
     {
