@@ -882,11 +882,14 @@ static hipError_t stream_product(hipStream_t st, FusedState *fs, int epi, const 
 
 // Prompt steps of small models whose widths the tile GEMM's epilogues do not take (D % 64 != 0, or heads that are not a
 // power of two of at least 32): five launches a layer (QKV with RoPE and the cache rows, attention, Wo + residual, gate
-// and up, down + residual), each product with the RMSNorm in front of it. Up to 256 tokens, the longest measured: the
-// tiny decoder (dim 288, 6 layers) 386 -> 197 us at 16 tokens; at 200 its kernels take 193 us instead of 417.
+// and up, down + residual), each product with the RMSNorm in front of it. us a step before and with it: tiny decoder (dim
+// 288, 6 layers) 16 tokens 386 / 197, 256 tokens 439 / 242; dim 992, 4 layers, 256 tokens 529 / 376. Longer steps were
+// measured with the vocabulary product here as well: 257 and 400 tokens are faster (dim 288, a vocabulary of 1000: 425 /
+// 249, 495 / 333), 1024 is slower (904 / 1004); between them the line is not placed, so it stays at the tiny decoder's cache.
 constexpr uint32_t kSmallPromptMax = 256;
-// the vocabulary product too while its 16 x 16 tiles are few enough that reading the weights once per 16 tokens is
-// nothing (a vocabulary of 1000); larger ones stay on the tile GEMM
+// The vocabulary product too up to this many 16 x 16 tiles: every 16 tokens read all of its weights. us a step with the
+// tile GEMM / with this kernel for 32000 words: 33 tokens (6000 tiles) 165 / 186 at dim 288 and 180 / 210 at 992, 128
+// tokens 182 / 222 and 266 / 358; 32 tokens (4000 tiles) at dim 992, all products on the tile GEMM 409, here 185.
 constexpr uint64_t kSmallLogitTiles = 4096;
 
 static bool prefill_small_ok(const ModelPriv *mp, uint32_t S)

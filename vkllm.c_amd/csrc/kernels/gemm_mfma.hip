@@ -7,8 +7,8 @@
 // K (described at the kernel). Its epilogue stages the tile's fp16 outputs in the freed LDS and stores 16-byte row chunks:
 // plain, SiLU on columns >= split, residual add, the FFN's up * silu(gate) (reading up and gate rows as interleaved
 // 16-row blocks), or the QKV product's RoPE with q and the K/V cache rows written directly.
-// gemm_kernel (other K): v_mfma_f32_16x16x32_f16, 128 x 128 or 128 x 64 tiles, the same double buffering, with the
-// K tail zeroed (plain, SiLU and residual epilogues only).
+// gemm_kernel (other K): v_mfma_f32_16x16x32_f16, 128 x 128 or 128 x 64 tiles, operands staged through registers into two
+// LDS buffers, with the K tail zeroed (plain, SiLU and residual epilogues only).
 //
 // Narrow products split K over several workgroups; the fp32 partial tiles are added in split order by
 // gemm_splitk_reduce_kernel, which applies the epilogue, or for a residual product followed by RMSNorm by
@@ -254,15 +254,14 @@ __host__ __device__ __forceinline__ void for_seq(std::integer_sequence<int, J...
     (f(std::integral_constant<int, J>{}), ...);
 }
 
-// n_base: product column of the kernel's column 0 (B rows and C columns are addressed from it; N counts the
-// kernel's columns). NH: halves in the LDS ring. WIDE: rows of any length, a tile's rows by 64-bit offsets (otherwise K <= kGemm32MaxK). Dual products read their columns from the up rows B and the gate rows B2 as interleaved 32-row
-// blocks and `split` holds F.
+// NH: halves in the LDS ring. WIDE: rows of any length, a tile's rows by 64-bit offsets (otherwise K <= kGemm32MaxK). Dual
+// products read their columns from the up rows B and the gate rows B2 as interleaved 16-row blocks and `split` holds F.
 template <int BM, int BN, int NH, int EPI, bool SPLIT, bool WIDE = false>
 __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                         const uint16_t *__restrict__ B2, uint16_t *C, float *work,
                                                         uint32_t M, uint32_t N, uint32_t K, uint32_t ldc,
                                                         uint32_t split, uint32_t kchunk, uint32_t tiles_m,
-                                                        uint32_t tiles_total, uint32_t n_base, GemmRope rope)
+                                                        uint32_t tiles_total, GemmRope rope)
 {
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
     constexpr int HALF = (BM + BN) * 64; // bytes of a half
@@ -284,8 +283,8 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
     // Copy i of a wave and half h fills the half's LDS rows 8 (wid + 4 i) .. + 7 (WM rows of A, then WN of B), lane l
     // row l / 8, chunk position l % 8. Rows past M or N repeat the last one: they only feed outputs that are not
     // stored. Every K step lies wholly inside [kb, ke) (the launcher admits whole 64-wide steps).
-    const uint32_t n_first = is_dual(EPI) ? (n_base + n0) / 2 : n_base + n0; // first row of B (and B2)
-    const uint32_t n_last = is_dual(EPI) ? split - 1 : n_base + N - 1;
+    const uint32_t n_first = is_dual(EPI) ? n0 / 2 : n0; // first row of B (and B2)
+    const uint32_t n_last = is_dual(EPI) ? split - 1 : N - 1;
     const char *const Ap = (const char *)(A + (size_t)m0 * K + kb);
     // dual products: waves 0 and 1 copy the up rows of each block, waves 2 and 3 its gate rows
     const char *const Bp = (const char *)((is_dual(EPI) && wid >= 2 ? B2 : B) + (size_t)n_first * K + kb);
@@ -441,15 +440,14 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
                             dual_out<EPI>(__uint_as_float(p[0]), __uint_as_float(p[1]));
                     }
                     else if constexpr (EPI == GEMM_SILU_HI)
-                        T[rt * TROW + ct] = f2h(n_base + n0 + ct >= split ? silu(acc[i][j][e]) : acc[i][j][e]);
+                        T[rt * TROW + ct] = f2h(n0 + ct >= split ? silu(acc[i][j][e]) : acc[i][j][e]);
                     else
                         T[rt * TROW + ct] = f2h(acc[i][j][e]);
                 }
         __syncthreads();
         constexpr int CH = OC / 8;
-        const uint32_t oc0 = is_dual(EPI) ? (n_base + n0) / 2 : n_base + n0; // output column of tile column 0
-        // end of this launch's columns
-        const uint32_t oce = is_dual(EPI) ? min((n_base + N) / 2, split) : n_base + N;
+        const uint32_t oc0 = is_dual(EPI) ? n0 / 2 : n0; // output column of tile column 0
+        const uint32_t oce = is_dual(EPI) ? split : N; // end of the output's columns
         const bool vec = ((uintptr_t)C % 16 == 0) && ldc % 8 == 0;
         if (vec && oc0 + OC <= oce)
         {
@@ -523,17 +521,17 @@ __global__ __launch_bounds__(256, 1) void gemm32_kernel(const uint16_t *__restri
             }
 }
 
-// C = epilogue(sum over z of work[z]) for split-K products, the splits added in order
 // whether the plain, SiLU and residual epilogues of the split-K reduce can move 8 columns as one 16-byte vector
-__host__ __device__ __forceinline__ bool reduce_vec8(uint32_t N, uint32_t ldc, uint32_t n_base, const uint16_t *C)
+__host__ __device__ __forceinline__ bool reduce_vec8(uint32_t N, uint32_t ldc, const uint16_t *C)
 {
-    return N % 8 == 0 && ldc % 8 == 0 && n_base % 8 == 0 && (uintptr_t)C % 16 == 0;
+    return N % 8 == 0 && ldc % 8 == 0 && (uintptr_t)C % 16 == 0;
 }
 
+// C = epilogue(sum over z of work[z]) for split-K products, the splits added in order
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *work, uint16_t *C, uint32_t M,
                                                                  uint32_t N, uint32_t ldc, uint32_t split,
-                                                                 uint32_t splits, uint32_t n_base, GemmRope rope)
+                                                                 uint32_t splits, GemmRope rope)
 {
     const uint64_t total = (uint64_t)M * N;
     // 8 consecutive columns per step (N % 64 == 0 for these epilogues): 16-byte partial loads and output stores
@@ -568,7 +566,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 h[k] = pack2(f2h(v[2 * k]), f2h(v[2 * k + 1]));
-            rope_store8(rope, m, n_base + n, h, rope_load8(rope, m, n_base + n));
+            rope_store8(rope, m, n, h, rope_load8(rope, m, n));
         }
         return;
     }
@@ -580,7 +578,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
         for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < chunks; i += (uint64_t)gridDim.x * 256)
         {
             const uint32_t m = (uint32_t)(i / per_row), f = 8 * (uint32_t)(i % per_row), c = 32 * (f / 16) + f % 16;
-            if (n_base / 2 + f >= split) // columns past F (GEMM_FFN with F % 32 != 0)
+            if (f >= split) // columns past F (GEMM_FFN with F % 32 != 0)
                 continue;
             float up[8], gate[8];
             sum8((size_t)m * N + c, up);
@@ -589,11 +587,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 o[k] = pack2(dual_out<EPI>(up[2 * k], gate[2 * k]), dual_out<EPI>(up[2 * k + 1], gate[2 * k + 1]));
-            *(u32x4 *)(C + (size_t)m * ldc + swiglu_col(n_base + c)) = o;
+            *(u32x4 *)(C + (size_t)m * ldc + swiglu_col(c)) = o;
         }
         return;
     }
-    if (reduce_vec8(N, ldc, n_base, C))
+    if (reduce_vec8(N, ldc, C))
     {
         // 8 consecutive columns per step: 16-byte partial loads and one 16-byte store (the same sums, in the same
         // split order, as the element loop below)
@@ -604,7 +602,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
             const uint32_t m = (uint32_t)(i / per_row), n = 8 * (uint32_t)(i % per_row);
             float v[8];
             sum8((size_t)m * N + n, v);
-            uint16_t *c = C + (size_t)m * ldc + n_base + n;
+            uint16_t *c = C + (size_t)m * ldc + n;
             u32x4 o;
             if constexpr (EPI == GEMM_RESID)
             {
@@ -618,7 +616,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
             {
 #pragma unroll
                 for (int k = 0; k < 8; ++k)
-                    if (EPI == GEMM_SILU_HI && n_base + n + k >= split)
+                    if (EPI == GEMM_SILU_HI && n + k >= split)
                         v[k] = silu(v[k]);
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
@@ -633,18 +631,18 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float *wo
         float v = 0.f;
         for (uint32_t z = 0; z < splits; ++z)
             v += work[(size_t)z * total + i];
-        gemm_store(EPI, C, ldc, (uint32_t)(i / N), n_base + (uint32_t)(i % N), v, split);
+        gemm_store(EPI, C, ldc, (uint32_t)(i / N), (uint32_t)(i % N), v, split);
     }
 }
 
 // work items of gemm_splitk_reduce_kernel: 8 columns each where the epilogue or reduce_vec8 allows, else one element
 template <int EPI>
-static uint32_t reduce_grid(uint32_t M, uint32_t N, uint32_t ldc, uint32_t n_base, const uint16_t *C)
+static uint32_t reduce_grid(uint32_t M, uint32_t N, uint32_t ldc, const uint16_t *C)
 {
     uint64_t items = (uint64_t)M * N;
     if (is_dual(EPI))
         items /= 16;
-    else if (EPI == GEMM_QKV_ROPE || reduce_vec8(N, ldc, n_base, C))
+    else if (EPI == GEMM_QKV_ROPE || reduce_vec8(N, ldc, C))
         items /= 8;
     const uint64_t grid = (items + 255) / 256;
     return (uint32_t)(grid > 4096 ? 4096 : grid < 1 ? 1 : grid);
@@ -819,7 +817,7 @@ static hipError_t launch_tile(hipStream_t st, const uint16_t *A, const uint16_t 
 template <int BM, int BN, int NH, int EPI, bool SPLIT, bool WIDE = false>
 static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, GemmB B, uint16_t *C, float *work,
                                 uint32_t M, uint32_t N, uint32_t K, uint32_t ldc, uint32_t split, uint32_t splits,
-                                uint32_t kchunk, uint32_t n_base = 0, const GemmRope *rope = nullptr)
+                                uint32_t kchunk, const GemmRope *rope = nullptr)
 {
     static uint64_t attr_devs = 0; // devices on which the LDS limit is raised for this kernel
     const size_t lds = (size_t)NH * (BM + BN) * 64;
@@ -829,17 +827,17 @@ static hipError_t launch_tile32(hipStream_t st, const uint16_t *A, GemmB B, uint
     const uint32_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, total = tm * tn;
     const uint32_t grid = (total + 7) / 8 * 8;
     gemm32_kernel<BM, BN, NH, EPI, SPLIT, WIDE><<<dim3(grid, SPLIT ? splits : 1), 256, lds, st>>>(
-        A, B.p, B.p2, C, work, M, N, K, ldc, split, kchunk, tm, total, n_base, rope ? *rope : GemmRope{});
+        A, B.p, B.p2, C, work, M, N, K, ldc, split, kchunk, tm, total, rope ? *rope : GemmRope{});
     return hipGetLastError();
 }
 
 template <int EPI>
 static hipError_t launch_reduce(hipStream_t st, const float *work, uint16_t *C, uint32_t M, uint32_t N, uint32_t ldc,
-                                uint32_t split, uint32_t splits, uint32_t n_base, const GemmRope *rope)
+                                uint32_t split, uint32_t splits, const GemmRope *rope)
 {
-    const uint32_t grid = reduce_grid<EPI>(M, N, ldc, n_base, C);
+    const uint32_t grid = reduce_grid<EPI>(M, N, ldc, C);
     gemm_splitk_reduce_kernel<EPI>
-        <<<grid, 256, 0, st>>>(work, C, M, N, ldc, split, splits, n_base, rope ? *rope : GemmRope{});
+        <<<grid, 256, 0, st>>>(work, C, M, N, ldc, split, splits, rope ? *rope : GemmRope{});
     return hipGetLastError();
 }
 
@@ -853,8 +851,8 @@ static hipError_t launch_shape(hipStream_t st, const uint16_t *A, const uint16_t
     hipError_t e = launch_tile<BM, BN, EPI, true>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk);
     if (e != hipSuccess)
         return e;
-    const uint32_t grid = reduce_grid<EPI>(M, N, ldc, 0, C);
-    gemm_splitk_reduce_kernel<EPI><<<grid, 256, 0, st>>>(work, C, M, N, ldc, split, splits, 0, GemmRope{});
+    const uint32_t grid = reduce_grid<EPI>(M, N, ldc, C);
+    gemm_splitk_reduce_kernel<EPI><<<grid, 256, 0, st>>>(work, C, M, N, ldc, split, splits, GemmRope{});
     return hipGetLastError();
 }
 
@@ -886,7 +884,7 @@ static hipError_t launch_choice(hipStream_t st, int tile, const uint16_t *A, Gem
     for_seq(std::make_integer_sequence<int, kTileCount>{}, [&](auto i) {
         constexpr TileShape T = kTiles[decltype(i)::value];
         if (tile == decltype(i)::value)
-            e = launch_tile32<T.bm, T.bn, T.ring, EPI, SPLIT>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, 0, rope);
+            e = launch_tile32<T.bm, T.bn, T.ring, EPI, SPLIT>(st, A, B, C, work, M, N, K, ldc, split, splits, kchunk, rope);
     });
     return e;
 }
@@ -900,8 +898,9 @@ struct TileChoice
 // Time of a product on one tile shape with K in `splits` ranges, us: the tile's measured step, or what the busy CUs
 // together sustain (1.3 PFLOP/s); each round of workgroups adds its start and its epilogue, split K the partials written
 // and read and the reduce's launch, whole K the RMSNorm pass that the reduce would have included; and the weights come
-// from HBM at 4.6 TB/s, or 24 bytes/ns of each workgroup (18 of a part of its rows). Over 73 products of 16 to 2048 rows at the 7B and 13B widths the choice made from it is the
-// fastest measured one or within 11% of it in all but 4.
+// from HBM at 4.6 TB/s, or 24 bytes/ns of each workgroup (18 of a part of its rows). Over 73 products of 16 to 2048 rows
+// at the 7B and 13B widths the choice made from it is the fastest measured one (of the eight tiles with a full ring and up
+// to 8 ranges) or within 11% of it in all but 2, which are within 14%.
 static float tile_time(uint32_t M, uint32_t N, uint32_t K, TileShape t, uint32_t splits, uint32_t cus, bool norm)
 {
     const uint64_t wgs = (uint64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * splits;
@@ -973,7 +972,8 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
         if (!rope || K % kBK != 0 || K > kGemm32MaxK || rope->D % 64 != 0 || rope->hd < 32 || (rope->hd & (rope->hd - 1)) != 0 ||
             N != 3 * rope->D || !rope->cs)
             return hipErrorInvalidValue;
-    if ((uint64_t)N * K >= (1ull << 32)) // B row offsets are 32-bit
+    // (no product past it has run: MATMUL refuses it too, the FFN operator takes its generic kernel)
+    if ((uint64_t)N * K >= (1ull << 32))
         return hipErrorInvalidValue;
     if constexpr (is_dual(EPI))
         if (K % kBK != 0 || (EPI == GEMM_FFN && K > kGemm32MaxK) || N % 64 != 0 || N != (2 * split + 63) / 64 * 64 ||
@@ -1001,7 +1001,7 @@ static hipError_t launch_epi_gemm(hipStream_t st, const uint16_t *A, GemmB B, ui
                 *normed = true;
                 return launch_resid_norm(st, work, C, M, N, splits, *norm);
             }
-        return launch_reduce<EPI>(st, work, C, M, N, ldc, split, splits, 0, rope);
+        return launch_reduce<EPI>(st, work, C, M, N, ldc, split, splits, rope);
     }
     if constexpr (is_dual(EPI) || EPI == GEMM_QKV_ROPE)
         return hipErrorInvalidValue; // checked above: not reached
@@ -1035,14 +1035,14 @@ hipError_t launch_gemm_reduce(hipStream_t st, int epi, const float *work, uint16
     {
     case GEMM_RESID:
         if (!norm)
-            return launch_reduce<GEMM_RESID>(st, work, C, M, N, N, 0, splits, 0, nullptr);
+            return launch_reduce<GEMM_RESID>(st, work, C, M, N, N, 0, splits, nullptr);
         if (N % 8 != 0 || (norm->xt && (M > 128 || N % 16 != 0)))
             return hipErrorInvalidValue;
         return launch_resid_norm(st, work, C, M, N, splits, *norm);
     case GEMM_QKV_ROPE:
         if (!rope || N != 3 * rope->D)
             return hipErrorInvalidValue;
-        return launch_reduce<GEMM_QKV_ROPE>(st, work, C, M, N, N, 0, splits, 0, rope);
+        return launch_reduce<GEMM_QKV_ROPE>(st, work, C, M, N, N, 0, splits, rope);
     default:
         return hipErrorInvalidValue;
     }

@@ -646,7 +646,7 @@ extern "C" vkllm_err_t vkllm_op_ffn_up_and_gate_init(struct vkllm_context *conte
 // fp16 operands in packed 16-byte-aligned rows run on the token step's kernels: one row on the streaming GEMV (K up to
 // the 22 vectors a lane holds of a row), more on the tile GEMM (K in whole 64-wide steps). Both sum in fp32 and round
 // the product once, as the generic kernel does. 7B widths: 512 rows 2756 us on the generic kernel (vector FMAs from
-// 64 x 64 LDS tiles), 119 us on the tile GEMM (92 GFLOP, 776 TFLOP/s; 172 of 256 CUs hold a tile); one row 27.7 us on
+// 64 x 64 LDS tiles), 90 us on the tile GEMM (92 GFLOP, 1.03 PFLOP/s; 232 tiles of 256 x 192 for 256 CUs); one row 27.7 us on
 // the GEMV, 6.5 TB/s of weights. Small products of other K (whole 32-wide steps) take the one-launch kernel of small
 // models: 16 rows of the tiny decoder's widths (288 to 768) 69 -> 3.3 us, 200 rows 81 -> 4.4.
 enum class FfnPath
